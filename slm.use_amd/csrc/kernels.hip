@@ -12,7 +12,7 @@
 //   - attend: keys are grouped by absolute position into 16-key tiles, 64-key segments
 //     and 256-key superblocks; a segment is an online softmax over its tiles, segments
 //     fold into superblocks in order and superblocks into the result in order;
-//   - gla: one kernel for every m, tokens in order;
+//   - gla: tokens in order, a column's sum one fixed tree over its rows;
 //   - rms / l2norm: the 16-accumulator dot of the reference CPU backend (src/cpu.rs:9-21),
 //     so these two are bit-identical to it;
 //   - the rest is element-wise.
@@ -113,6 +113,49 @@ __device__ __forceinline__ bool step_wait(const StepWait& w, int lane) {
     if (gave_up) wait_gave_up(w.fault, lane);
     return gave_up;
 }
+
+template <int N>
+__device__ __forceinline__ void vm_wait() {  // s_waitcnt vmcnt(N), other counters untouched
+    static_assert(N >= 0 && N < 64, "vmcnt");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// Sixteen zero bytes: what a lane past the end of its operand loads.
+__device__ __attribute__((aligned(16))) float slm_zero16[4];
+
+// v combined with lane l ^ 16 (or l ^ 32) through register lane swaps: v_permlane16_swap
+// gives every lane its row pair's even-row and odd-row values (v_permlane32_swap its half
+// pair's), so a symmetric op of the two is the lane's value with its partner's — the same bits
+// as op(v, shfl_xor(v, 16)) for the commutative max, + and |.
+__device__ __forceinline__ float xmax16(float v) {
+    auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+__device__ __forceinline__ float xmax32(float v) {
+    auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+__device__ __forceinline__ float xsum16(float v) {
+    auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float xsum32(float v) {
+    auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ int xor16i(int v) {
+    auto p = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    return (int)(p[0] | p[1]);
+}
+__device__ __forceinline__ int xor32i(int v) {
+    auto p = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    return (int)(p[0] | p[1]);
+}
+
+template <bool V>
+struct Flag {
+    static constexpr bool value = V;
+};
 
 // A workgroup barrier that orders LDS only (what memory loads are in flight stay in flight).
 __device__ __forceinline__ void lds_bar() {
@@ -517,373 +560,344 @@ KERNEL void __launch_bounds__(256) slm_l2norm(float* y, const float* x, int grou
 // gated linear attention (ops.rs:191-205, cpu.rs:284-329)
 // ---------------------------------------------------------------------------------------
 //
-// Sixteen lanes per state column b (lanes 16c .. 16c+15 of a wave); lane j owns rows
-// j·RPL .. j·RPL+RPL-1 of S[h][:, b] in registers. Tokens run in order:
-// d = 1/(1 + e^(decay + bias)), S[a][b] = d·S[a][b] + k[a]·v[b], y[b] = Σ_a q[a]·S[a][b],
-// where each lane sums its rows in order and the sixteen lane sums are added pairwise
-// by lane distance 1, 2, 4, 8 (gla_colsum). The prompt kernel and the one-token kernel
-// (gla1_body) run the same expressions.
+// A state column S[h][:, b] is summed as a fixed tree over its rows, padded with zeros to
+// P = 16, 32, 64, 128 or 256 (the next size that holds dh): row distances P/2, P/4, .. 8 by
+// pairs (a, a + distance), then within the eight sums left (i, 7 - i), then distance 2 and 1.
+// Tokens run in order: d = 1/(1 + e^(decay + bias)), S[a][b] = d·S[a][b] + k[a]·v[b],
+// y[b] = Σ_a q[a]·S[a][b]. The prompt kernel and the one-token kernel (gla1_body) run the same
+// expressions; the tree is what both can form with register lane swaps only.
 
-// xor-1 and xor-2 lane swaps within quads (DPP quad_perm [1,0,3,2] and [2,3,0,1])
-__device__ __forceinline__ float dpp_xor1(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xF, 0xF, false));
+// Lane swaps within rows of sixteen (DPP): i ^ 8, i ^ 7 within eights, i ^ 2, i ^ 1.
+template <int CTRL>
+__device__ __forceinline__ float dpp_swap(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
 }
-__device__ __forceinline__ float dpp_xor2(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4E, 0xF, 0xF, false));
-}
-// The column total of the sixteen lane sums, in every lane of the sixteen.
+constexpr int DPP_X8 = 0x128, DPP_X7 = 0x141, DPP_X2 = 0x4E, DPP_X1 = 0xB1;
+
+// The total of sixteen lanes' values, in every lane of the sixteen (the tree's last levels).
 __device__ __forceinline__ float gla_colsum(float p) {
-    p = p + dpp_xor1(p);
-    p = p + dpp_xor2(p);
-    p = p + __shfl_xor(p, 4);
-    p = p + __shfl_xor(p, 8);
+    p = p + dpp_swap<DPP_X8>(p);
+    p = p + dpp_swap<DPP_X7>(p);
+    p = p + dpp_swap<DPP_X2>(p);
+    p = p + dpp_swap<DPP_X1>(p);
     return p;
 }
 
-// The same total in the column's first lane only (what the prompt kernel stores): distance
-// 4 and 8 through DPP row shifts (lane 16c + i reads lane 16c + i + n), so lane 16c adds the
-// same pairs in the same order as gla_colsum. (Lanes whose source is past the row read zero,
-// bound_ctrl, which lets each shift fuse into its add; only lane 16c's total is used, and its
-// sources are always inside the row.)
-__device__ __forceinline__ float gla_colsum0(float p) {
-    p = p + dpp_xor1(p);
-    p = p + dpp_xor2(p);
-    p = p + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(p), 0x104, 0xF, 0xF, true));
-    p = p + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(p), 0x108, 0xF, 0xF, true));
-    return p;
-}
-
-// One lane's rows for one token: st = d·st + k·v, and the lane's sum of q·st in order.
-// One state element's update for one token, st·d + k·v (fp16 mode: mlx.rs:321's state.multiply,
+// One state element's update for one token, st·d + k·v, the first product unrounded (fp16 mode: mlx.rs:321's state.multiply,
 // ki.multiply and add, each rounded); and the decay factor sigmoid(−(raw + bias)) (mlx.rs:313).
 template <bool H>
 __device__ __forceinline__ float gla_upd(float dc, float s, float k, float v) {
-    return H ? r16(r16(dc * s) + r16(k * v)) : dc * s + k * v;
+    return H ? r16(r16(dc * s) + r16(k * v)) : fmaf(dc, s, k * v);
 }
 template <bool H>
 __device__ __forceinline__ float gla_decay(float raw, float bias) {
     return H ? r16(1.0f / (1.0f + expf(r16(raw + bias)))) : 1.0f / (1.0f + expf(raw + bias));
 }
 
-template <int RPL, bool H = false>
+// The tree's levels inside a lane that holds N rows a whole number of levels apart.
+template <int N>
+__device__ __forceinline__ float gla_tree(float (&p)[N]) {
+#pragma unroll
+    for (int n = N / 2; n > 0; n /= 2)
+#pragma unroll
+        for (int r = 0; r < n; r++) p[r] = p[r] + p[r + n];
+    return p[0];
+}
+
+// One token for a lane of the one-token kernel, which holds rows j, j + 16, ... of a column:
+// the state's update and the lane's part of the column's sum.
+template <int RPL, bool H>
 __device__ __forceinline__ float gla_rows(float (&st)[RPL], const float* kk, const float* qq,
                                           float dc, float vb, int j, int dh) {
-    float part = 0.0f;
-    if ((j + 1) * RPL <= dh) {
+    float p[RPL], kv[RPL], qv[RPL];
 #pragma unroll
-        for (int rr = 0; rr < RPL; rr++) {
-            int a = j * RPL + rr;
-            st[rr] = gla_upd<H>(dc, st[rr], kk[a], vb);
-            part = part + qq[a] * st[rr];
-        }
-    } else {
-#pragma unroll
-        for (int rr = 0; rr < RPL; rr++) {
-            int a = j * RPL + rr;
-            if (a < dh) {
-                st[rr] = gla_upd<H>(dc, st[rr], kk[a], vb);
-                part = part + qq[a] * st[rr];
-            }
-        }
+    for (int rr = 0; rr < RPL; rr++) {  // (no branches: every read is out before the first use)
+        int a = min(j + 16 * rr, dh - 1);
+        kv[rr] = kk[a];
+        qv[rr] = qq[a];
     }
-    return part;
-}
-
-// gla_rows when every lane's RPL rows are inside the head: the rows' k and q read as float4s.
-template <int RPL, bool H = false>
-__device__ __forceinline__ float gla_rows_full(float (&st)[RPL], const float* kk, const float* qq,
-                                               float dc, float vb, int j) {
-    float kv[RPL], qv[RPL];
-    if constexpr (RPL % 4 == 0) {
-#pragma unroll
-        for (int c = 0; c < RPL / 4; c++) {
-            f4 a = *(const f4*)(kk + j * RPL + 4 * c), b = *(const f4*)(qq + j * RPL + 4 * c);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                kv[4 * c + e] = a[e];
-                qv[4 * c + e] = b[e];
-            }
-        }
-    } else {
-#pragma unroll
-        for (int rr = 0; rr < RPL; rr++) {
-            kv[rr] = kk[j * RPL + rr];
-            qv[rr] = qq[j * RPL + rr];
-        }
-    }
-    float part = 0.0f;
 #pragma unroll
     for (int rr = 0; rr < RPL; rr++) {
-        st[rr] = gla_upd<H>(dc, st[rr], kv[rr], vb);
-        part = part + qv[rr] * st[rr];
+        float s = gla_upd<H>(dc, st[rr], kv[rr], vb);
+        bool in = j + 16 * rr < dh;
+        st[rr] = in ? s : st[rr];
+        p[rr] = in ? qv[rr] * s : 0.0f;
     }
-    return part;
+    return gla_tree<RPL>(p);
 }
 
-// One token's operands for a lane of the prompt kernel's pipelined path: its RPL rows of k
-// and q and the column's v.
-template <int RPL>
-struct GlaOps {
-    float k[RPL], q[RPL], v;
+// Two tokens' partial sums a, b into one register, one tree level further: lanes whose bit M
+// is clear keep a's sums, the others b's (CTRL swaps lanes that differ in bit M).
+template <int M, int CTRL>
+__device__ __forceinline__ float gla_merge(float a, float b, int lane) {
+    bool hi = (lane & M) != 0;
+    return (hi ? b : a) + dpp_swap<CTRL>(hi ? a : b);
+}
+
+// The prompt kernel: a wave holds one column of a head's state, a lane one row of it (P > 64:
+// rows lane + 64·r; P < 64: 64 / P columns a wave), four waves a workgroup, grid (heads,
+// groups of 4 columns or 4·64/P). What bounds it is the issue rate of each wave's token loop,
+// tokens being serial: sixteen lanes a column with four rows each ran about 30 instructions a
+// token on 192 waves (12 heads of 64); one row a lane runs about 9 on 768, so most of the chip
+// works on it. The column sums are taken for sixteen tokens at once: each tree level joins two
+// tokens' registers (lane swaps and selects), so a token's six levels cost about two
+// instructions, and its output leaves in one store with the fifteen others'.
+// k, q and v rows and decay inputs arrive in a ring of four LDS stages of T tokens by direct
+// copies, two stages in flight while one is used; each stage's (v, d) pairs are made one stage
+// ahead. 256 tokens, 12 heads of 64: 25.6 -> 11.4 us a call.
+template <int P, bool H>
+struct GlaShape {
+    static constexpr int RPL = P > 64 ? P / 64 : 1;      // rows a lane
+    static constexpr int LPC = P < 64 ? P : 64;          // lanes a column
+    static constexpr int NC = 4 * (64 / LPC);            // columns a workgroup
+    static constexpr int T = P > 64 ? 16 : 32;           // tokens a stage
+    static constexpr int KQ = T * 2 * P;                 // a stage's [T][k (P) | q (P)]
+    static constexpr int NVI = (T * (NC + 1) + 255) / 256;  // copies a wave of v and decay inputs
+    static constexpr int STAGE = KQ + 256 * NVI;         // floats: then [T][NC] v, [T] decay inputs
+    static constexpr int STAGES = 4;
+    static constexpr int LDS = STAGES * STAGE + 2 * NC * T * 2;  // then two [NC][T] (v, d)
 };
-// gla_rows_full's expressions on operands already in registers.
-template <int RPL>
-__device__ __forceinline__ float gla_step(float (&st)[RPL], const GlaOps<RPL>& o, float dc) {
-    float part = 0.0f;
-#pragma unroll
-    for (int rr = 0; rr < RPL; rr++) {
-        st[rr] = dc * st[rr] + o.k[rr] * o.v;
-        part = part + o.q[rr] * st[rr];
-    }
-    return part;
-}
-
-// The prompt kernel: grid (heads, groups of SLM_GLA_COLS columns), one wave a workgroup (so a
-// CU's LDS serves one wave's reads); each workgroup stages q and k of its head and v of its
-// columns for SLM_GLA_T tokens at a time in LDS.
-template <int RPL, bool H>
-__device__ void gla_body(float* __restrict__ y, float* __restrict__ S,
+template <int P, bool H>
+__device__ __forceinline__ void gla_body(float* __restrict__ y, float* __restrict__ S,
                          const float* __restrict__ q, const float* __restrict__ k,
                          const float* __restrict__ v, const float* __restrict__ decay,
                          const float* __restrict__ bias, int m, int heads, int dh, int vec) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];  // 2 x ([SLM_GLA_T][q (dh) | k (dh) | v (SLM_GLA_COLS)], then [SLM_GLA_T] d)
-    constexpr int NC = SLM_GLA_COLS;
-    int h = blockIdx.x, c0 = blockIdx.y * NC, tid = threadIdx.x, nt = blockDim.x;
-    int b = c0 + (tid >> 4), j = tid & 15;
+    using G = GlaShape<P, H>;
+    constexpr int RPL = G::RPL, LPC = G::LPC, NC = G::NC, T = G::T, B = 16;
+    static_assert(T % B == 0 && G::LDS * 4 <= 160 * 1024, "whole blocks of tokens, LDS of a CU");
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int h = blockIdx.x, c0 = blockIdx.y * NC;
+    int cw = wave * (64 / LPC) + lane / LPC, a0 = lane % LPC, b = c0 + cw;
     bool live = b < dh;
     float* Sh = S + (long long)h * dh * dh;
     float st[RPL];
 #pragma unroll
     for (int rr = 0; rr < RPL; rr++) {
-        int a = j * RPL + rr;
+        int a = a0 + 64 * rr;
         st[rr] = (live && a < dh) ? Sh[(long long)a * dh + b] : 0.0f;
     }
     float bh = bias[h];
-    bool full = 16 * RPL == dh && c0 + NC <= dh;  // uniform
-    int rowl = 2 * dh + NC, bufl = SLM_GLA_T * (rowl + 1);
-    // Two LDS buffers of SLM_GLA_T token rows (then their decays): the next group's rows are
-    // copied straight into one (and its decay inputs loaded into registers) while the
-    // tokens of the other run. Thread tid copies piece pc (of `vec` floats) of tokens
-    // tt0, tt0 + tpar, ...: piece tid·vec of the buffer, so a wave's copies are contiguous.
-    // (A row longer than the workgroup, lpt > nt: thread tid copies pieces tid, tid + nt, ...
-    // of every token instead.)
-    int lpt = rowl / vec, tpar = max(1, nt / lpt);
-    int tt0 = tid / lpt, pc = (tid % lpt) * vec;
-    bool loader = tid < tpar * lpt;
-    auto piece_src = [&](int pf) {  // token 0's source of the piece at float pf of a row
-        const float* sp = q + (long long)h * dh;  // (a piece past the head's columns copies q)
-        if (pf < dh) sp = q + (long long)h * dh + pf;
-        else if (pf < 2 * dh) sp = k + (long long)h * dh + pf - dh;
-        else if (c0 + pf - 2 * dh < dh) sp = v + (long long)h * dh + c0 + pf - 2 * dh;
-        return sp;
+    float2* pairs = (float2*)(lds + G::STAGES * G::STAGE);
+    const long long ts = (long long)heads * dh;  // token stride
+    int ng = (m + T - 1) / T;
+    // Copies of group g into its stage. Rows past dh and columns past it copy zeros, tokens
+    // past m the last token again (they are not used), so every wave issues the same number.
+    auto copy4 = [&](const float* src, float* dst) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                         (__attribute__((address_space(3))) void*)dst, 4, 0, 0);
     };
-    const float* src0 = piece_src(pc);
-    int wbase = (tid & ~63) * vec;  // this wave's first piece
-    auto copy = [&](const float* src, float* dst) {
-        if (vec == 4)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                             (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-        else
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                             (__attribute__((address_space(3))) void*)dst, 4, 0, 0);
+    auto copy16 = [&](const float* src, float* dst) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                         (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
     };
-    auto issue = [&](int i0, int buf) {
-        int nt_tok = min(SLM_GLA_T, m - i0);
-        float* base = lds + buf * bufl + wbase;
-        if (lpt > nt) {
-            for (int tt = 0; tt < nt_tok; tt++)
-                for (int r = 0; r * nt < lpt; r++)
-                    if (r * nt + tid < lpt)
-                        copy(piece_src((r * nt + tid) * vec) + (long long)(i0 + tt) * heads * dh,
-                             base + tt * rowl + r * nt * vec);
-            return;
+    // (a thread's pieces have one source and one token stride: selected once, so the copies
+    // themselves are unconditional)
+    constexpr int PT = 2 * P / 4;  // 16-byte pieces a token: PT threads each
+    const float* src[2];
+    int step[2];
+#pragma unroll
+    for (int z = 0; z < 2; z++) {  // (single floats at P = 256: one row of k, then one of q)
+        int o = vec == 4 ? 4 * (tid % PT) : (tid + 256 * z) % (2 * P);
+        const float* row = (o < P ? k : q) + (long long)h * dh;
+        o = o < P ? o : o - P;
+        src[z] = o < dh ? row + o : slm_zero16;
+        step[z] = o < dh ? heads * dh : 0;
+    }
+    const float* vsrc[G::NVI];
+    int vstep[G::NVI], vtok[G::NVI];
+#pragma unroll
+    for (int r = 0; r < G::NVI; r++) {
+        int e = r * 256 + tid, c = e % NC;
+        bool dec = e >= T * NC, in = dec ? e < T * (NC + 1) : c0 + c < dh;
+        vsrc[r] = !in ? slm_zero16 : dec ? decay + h : v + (long long)h * dh + c0 + c;
+        vstep[r] = !in ? 0 : dec ? heads : heads * dh;
+        vtok[r] = dec ? e - T * NC : e / NC;
+    }
+    auto issue = [&](int g) {
+        float* base = lds + (g % G::STAGES) * G::STAGE;
+        int i0 = g * T;
+        if (vec == 4) {
+#pragma unroll
+            for (int r = 0; r < G::KQ / 1024; r++) {
+                int tt = min(i0 + tid / PT + r * (256 / PT), m - 1);
+                copy16(src[0] + (long long)tt * step[0], base + r * 1024 + wave * 256);
+            }
+        } else {
+#pragma unroll 4
+            for (int r = 0; r < G::KQ / 256; r++) {
+                int z = P == 256 ? r & 1 : 0;
+                int tt = min(i0 + (r * 256 + tid) / (2 * P), m - 1);
+                copy4((z ? src[1] : src[0]) + (long long)tt * (z ? step[1] : step[0]), base + r * 256 + wave * 64);
+            }
         }
-        if (!loader) return;
-        // tokens tt0, tt0 + tpar, ...: the source and destination advance by fixed strides
-        const float* src = src0 + (long long)(i0 + tt0) * heads * dh;
-        const long long sstep = (long long)tpar * heads * dh;
-        float* dst = base;
-        const int dstep = tpar * rowl;
-        if (vec == 4)
-            for (int tt = tt0; tt < nt_tok; tt += tpar, src += sstep, dst += dstep)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                                 (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-        else
-            for (int tt = tt0; tt < nt_tok; tt += tpar, src += sstep, dst += dstep)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                                 (__attribute__((address_space(3))) void*)dst, 4, 0, 0);
-    };
-    float dnext = 0.0f;  // thread tt: the decay input of token tt of the next group
-    issue(0, 0);
-    if (tid < min(SLM_GLA_T, m)) dnext = decay[(long long)tid * heads + h];
-    // The outputs of a pipelined group's last eight tokens are stored only after the next
-    // group's copies are issued, so that the wait for those copies does not also wait for
-    // stores issued just before it.
-    float pend[8];
-    float* pend_y = nullptr;  // (the first of the eight tokens' outputs of this lane's column)
-    const int ys = heads * dh;  // token stride of y
-    auto store_pend = [&]() {
-        if (pend_y && j == 0)
 #pragma unroll
-            for (int u = 0; u < 8; u++) pend_y[u * ys] = pend[u];
-        pend_y = nullptr;
-    };
-    for (int i0 = 0, buf = 0; i0 < m; i0 += SLM_GLA_T, buf ^= 1) {
-        int nt_tok = min(SLM_GLA_T, m - i0);
-        const float* rows = lds + buf * bufl;
-        float* dcs = lds + buf * bufl + SLM_GLA_T * rowl;
-        __builtin_amdgcn_s_waitcnt(0);  // this thread's copies of the group are in
-        if (tid < nt_tok) dcs[tid] = gla_decay<H>(dnext, bh);
-        // every thread's copies and decays are in, and every thread is done with the group
-        // before (whose buffer the next copies overwrite)
-        __syncthreads();
-        if (i0 + SLM_GLA_T < m) {
-            issue(i0 + SLM_GLA_T, buf ^ 1);
-            if (tid < min(SLM_GLA_T, m - i0 - SLM_GLA_T)) dnext = decay[(long long)(i0 + SLM_GLA_T + tid) * heads + h];
+        for (int r = 0; r < G::NVI; r++) {
+            int tt = min(i0 + vtok[r], m - 1);
+            copy4(vsrc[r] + (long long)tt * vstep[r], base + G::KQ + r * 256 + wave * 64);
         }
-        store_pend();
-        // eight tokens at a time: their state updates in order, then their eight column
-        // sums side by side (no token's sum waits for the next token's update)
-        if constexpr (RPL <= 8) if (full && nt_tok == SLM_GLA_T) {
-            // every lane's rows inside the head (dh = 16·RPL), every column live, a whole
-            // group: the operands of token t + 2 are read from LDS while token t runs (four
-            // register sets in turn), so no token waits for its reads; each read is a lane
-            // base plus a constant offset
-            constexpr int DH = 16 * RPL, ROWL = 2 * DH + NC;
-            const float* qb = rows + j * RPL;
-            const float* vb = rows + 2 * DH + (b - c0);
-            // LDS reads per token (k and q rows, v); a token's reads are in once at most the two
-            // later tokens' reads are pending
-            constexpr int GLA_NRD = (RPL % 4 == 0 ? RPL / 2 : 2 * RPL) + 1;
-            constexpr int GLA_WAIT = 2 * GLA_NRD < 15 ? 2 * GLA_NRD : 15;
-            GlaOps<RPL> ops[4];
-            auto load = [&](GlaOps<RPL>& o, int t) {
-                if constexpr (RPL % 4 == 0) {
+    };
+    // Group g's (v, d) pairs, from its raw stage
+    auto make_pairs = [&](int g) {
+        const float* raw = lds + (g % G::STAGES) * G::STAGE + G::KQ;
+        float2* pr = pairs + (g & 1) * NC * T;
 #pragma unroll
-                    for (int c = 0; c < RPL / 4; c++) {
-                        f4 ka = *(const f4*)(qb + t * ROWL + DH + 4 * c), qa = *(const f4*)(qb + t * ROWL + 4 * c);
+        for (int e = tid; e < NC * T; e += 256) {
+            int c = e / T, t = e % T;
+            pr[e] = float2{raw[t * NC + c], gla_decay<H>(raw[T * NC + t], bh)};
+        }
+    };
+    // (no fence: the copies in flight go on; the wave's LDS accesses are done)
+    auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    constexpr int NCOPY = G::KQ / 1024 + G::NVI;  // a wave's copies a stage (vec 4)
+    static_assert(2 * NCOPY < 64, "copies the counter holds");
 #pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            o.k[4 * c + e] = ka[e];
-                            o.q[4 * c + e] = qa[e];
-                        }
-                    }
-                } else {
+    for (int g = 0; g < G::STAGES - 1; g++) issue(g);  // (past the last group: its last token again)
+    if (vec == 4) vm_wait<2 * NCOPY>();
+    else vm_wait<0>();
+    barrier();
+    make_pairs(0);
+    auto run = [&](auto full) {
+        constexpr bool FULL = decltype(full)::value;  // dh = P: every row inside the head
+        for (int g = 0; g < ng; g++) {
+            // group g + 1 is in (its pairs are made below) and every wave is done with group
+            // g - 1, whose stage group g + 3 takes
+            if (vec == 4 && g + 2 < ng) vm_wait<NCOPY>();
+            else vm_wait<0>();
+            barrier();
+            if (g + 3 < ng) issue(g + 3);
+            if (g + 1 < ng) make_pairs(g + 1);
+            const float* kq = lds + (g % G::STAGES) * G::STAGE + a0;
+            const float2* pr = pairs + ((g & 1) * NC + cw) * T;
+            int nt = min(T, m - g * T);
+            float* yg = y + (long long)g * T * ts + (long long)h * dh + b;
+            // a token's update and the lane's part of its sum
+            auto token = [&](const float* kk, const float* qq, float vt, float dt) {
+                float p[RPL];
+#pragma unroll
+                for (int rr = 0; rr < RPL; rr++) {
+                    st[rr] = gla_upd<H>(dt, st[rr], kk[rr], vt);
+                    p[rr] = qq[rr] * st[rr];
+                    if (!FULL && a0 + 64 * rr >= dh) st[rr] = p[rr] = 0.0f;
+                }
+                return gla_tree<RPL>(p);
+            };
+            // sixteen tokens' operands, read from LDS before the arithmetic of the tokens before
+            struct Blk {
+                float k[B][RPL], q[B][RPL];
+                f4 vd[B / 2];
+            };
+            auto load = [&](Blk& o, int t0) {
+#pragma unroll
+                for (int u = 0; u < B; u++) {
+                    if (u % 2 == 0) o.vd[u / 2] = *(const f4*)(pr + t0 + u);
 #pragma unroll
                     for (int rr = 0; rr < RPL; rr++) {
-                        o.k[rr] = qb[t * ROWL + DH + rr];
-                        o.q[rr] = qb[t * ROWL + rr];
+                        o.k[u][rr] = kq[(t0 + u) * 2 * P + 64 * rr];
+                        o.q[u][rr] = kq[(t0 + u) * 2 * P + P + 64 * rr];
                     }
                 }
-                o.v = vb[t * ROWL];
             };
-            // the group's decay factors, read once (four at a time: the decays start 16-byte
-            // aligned, as SLM_GLA_T is a multiple of 4)
-            static_assert(SLM_GLA_T % 8 == 0, "the prompt GLA runs whole blocks of eight tokens");
-            float dg[SLM_GLA_T];
+            auto block = [&](const Blk& o, int t0) {
+                float p[B];
 #pragma unroll
-            for (int t = 0; t < SLM_GLA_T; t += 4) {
-                f4 d4 = *(const f4*)(dcs + t);
+                for (int u = 0; u < B; u++)
+                    p[u] = token(o.k[u], o.q[u], o.vd[u / 2][2 * (u % 2)], o.vd[u / 2][2 * (u % 2) + 1]);
+                // sixteen tokens' sums, a register's lanes shared by twice as many tokens a level
+                int n = B;
+                if constexpr (LPC == 64) {
+                    n /= 2;
 #pragma unroll
-                for (int e = 0; e < 4; e++) dg[t + e] = d4[e];
-            }
-            __builtin_amdgcn_s_waitcnt(0xC07F);  // (nothing pending: the counts below are exact)
-#pragma unroll
-            for (int u = 0; u < 2; u++) load(ops[u], u);
-            // step t updates the state with token t and sums token t - 1 over the state that
-            // token left (the same expressions as gla_rows_full, in two halves that do not
-            // wait for each other)
-            float part[8];
-            float* yg = y + ((long long)i0 * heads + h) * dh + b;  // token i0's output, column b
-#pragma unroll
-            for (int t = 0; t <= SLM_GLA_T; t++) {
-                if (t < SLM_GLA_T) {
-                    // (past the group's last token the last row is read again, unused)
-                    load(ops[(t + 2) & 3], min(t + 2, SLM_GLA_T - 1));
-                    __builtin_amdgcn_s_waitcnt(0xC07F | (GLA_WAIT << 8));
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                float sn[RPL];
-                if (t < SLM_GLA_T) {
-                    const GlaOps<RPL>& o = ops[t & 3];
-#pragma unroll
-                    for (int rr = 0; rr < RPL; rr++) sn[rr] = gla_upd<H>(dg[t], st[rr], o.k[rr], o.v);
-                }
-                if (t > 0) {
-                    const GlaOps<RPL>& o = ops[(t - 1) & 3];
-                    float pp = 0.0f;
-#pragma unroll
-                    for (int rr = 0; rr < RPL; rr++) pp = pp + o.q[rr] * st[rr];
-                    part[(t - 1) & 7] = pp;
-                }
-                if (t < SLM_GLA_T)
-#pragma unroll
-                    for (int rr = 0; rr < RPL; rr++) st[rr] = sn[rr];
-                __builtin_amdgcn_sched_barrier(0);
-                if (t > 0 && (t & 7) == 0) {
-#pragma unroll
-                    for (int u = 0; u < 8; u++) part[u] = h16<H>(gla_colsum0(part[u]));
-                    if (t == SLM_GLA_T) {
-#pragma unroll
-                        for (int u = 0; u < 8; u++) pend[u] = part[u];
-                        pend_y = yg + (t - 8) * ys;
-                    } else if (j == 0) {
-#pragma unroll
-                        for (int u = 0; u < 8; u++) yg[(t - 8 + u) * ys] = part[u];
+                    for (int u = 0; u < n; u++) {
+                        auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[u]), __float_as_uint(p[u + n]), false, false);
+                        p[u] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
                     }
                 }
-            }
-            continue;
-        }
-        for (int t0 = 0; t0 < nt_tok; t0 += 8) {
-            int nu = min(8, nt_tok - t0);
-            float part[8];
-            if (full && nu == 8) {  // (every lane's rows inside the head, every column live)
+                if constexpr (LPC >= 32) {
+                    n /= 2;
 #pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    const float* row = rows + (t0 + u) * rowl;
-                    part[u] = gla_rows_full<RPL, H>(st, row + dh, row, dcs[t0 + u], row[2 * dh + (b - c0)], j);
-                }
-            } else {
-#pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    part[u] = 0.0f;
-                    if (u < nu && live) {
-                        const float* row = rows + (t0 + u) * rowl;
-                        part[u] = gla_rows<RPL, H>(st, row + dh, row, dcs[t0 + u], row[2 * dh + (b - c0)], j, dh);
+                    for (int u = 0; u < n; u++) {
+                        auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(p[u]), __float_as_uint(p[u + n]), false, false);
+                        p[u] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
                     }
                 }
+                n /= 2;
+#pragma unroll
+                for (int u = 0; u < n; u++) p[u] = gla_merge<8, DPP_X8>(p[u], p[u + n], lane);
+                n /= 2;
+#pragma unroll
+                for (int u = 0; u < n; u++) p[u] = gla_merge<4, DPP_X7>(p[u], p[u + n], lane);
+                float tot;
+                if constexpr (LPC == 64) {
+                    tot = p[0] + dpp_swap<DPP_X2>(p[0]);
+                    tot = tot + dpp_swap<DPP_X1>(tot);
+                } else if constexpr (LPC == 32) {
+                    tot = gla_merge<2, DPP_X2>(p[0], p[1], lane);
+                    tot = tot + dpp_swap<DPP_X1>(tot);
+                } else {
+                    p[0] = gla_merge<2, DPP_X2>(p[0], p[2], lane);
+                    p[1] = gla_merge<2, DPP_X2>(p[1], p[3], lane);
+                    tot = gla_merge<1, DPP_X1>(p[0], p[1], lane);
+                }
+                // the lane's token: its bits from the first level merged down
+                constexpr int SH = LPC == 64 ? 2 : LPC == 32 ? 1 : 0;
+                int tok = t0 + ((lane & (LPC - 1)) >> SH);
+                if (live && (lane & ((1 << SH) - 1)) == 0) yg[tok * ts] = h16<H>(tot);
+            };
+            int t0 = 0;
+            if (nt == T) {
+                Blk x[T / B];
+#pragma unroll
+                for (int z = 0; z < T / B; z++) load(x[z], z * B);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int z = 0; z < T / B; z++) block(x[z], z * B);
+                t0 = T;
+            } else if (nt >= B) {
+                Blk x;
+                load(x, 0);
+                block(x, 0);
+                t0 = B;
             }
+            for (; t0 < nt; t0++) {  // the last tokens one at a time: the same tree
+                float kk[RPL], qq[RPL];
 #pragma unroll
-            for (int u = 0; u < 8; u++) part[u] = h16<H>(gla_colsum0(part[u]));
-            if (live && j == 0)
-#pragma unroll
-                for (int u = 0; u < 8; u++)
-                    if (u < nu) y[((long long)(i0 + t0 + u) * heads + h) * dh + b] = part[u];
+                for (int rr = 0; rr < RPL; rr++) {
+                    kk[rr] = kq[t0 * 2 * P + 64 * rr];
+                    qq[rr] = kq[t0 * 2 * P + P + 64 * rr];
+                }
+                float p = token(kk, qq, pr[t0].x, pr[t0].y);
+                if constexpr (LPC == 64) p = xsum32(p);
+                if constexpr (LPC >= 32) p = xsum16(p);
+                p = gla_colsum(p);
+                if (live && a0 == 0) yg[t0 * ts] = h16<H>(p);
+            }
         }
-    }
-    store_pend();
+    };
+    if (dh == P) run(Flag<true>{});
+    else run(Flag<false>{});
+    vm_wait<0>();  // (a short call's copies past its last group)
 #pragma unroll
     for (int rr = 0; rr < RPL; rr++) {
-        int a = j * RPL + rr;
+        int a = a0 + 64 * rr;
         if (live && a < dh) Sh[(long long)a * dh + b] = st[rr];
     }
 }
 
 // (slm_glah_*: fp16 mode's)
-#define GLA_K(NAME, R, H)                                                              \
-    KERNEL void __launch_bounds__(16 * SLM_GLA_COLS)                                    \
+#define GLA_K(NAME, P, H)                                                              \
+    KERNEL void __launch_bounds__(256)                                                 \
         NAME(float* y, float* S, const float* q, const float* k, const float* v,        \
              const float* decay, const float* bias, int m, int heads, int dh,           \
              int vec) {                                                                 \
-        gla_body<R, H>(y, S, q, k, v, decay, bias, m, heads, dh, vec);                  \
+        gla_body<P, H>(y, S, q, k, v, decay, bias, m, heads, dh, vec);                  \
     }
-#define GLA(R) GLA_K(slm_gla_##R, R, false) GLA_K(slm_glah_##R, R, true)
-GLA(1)
-GLA(2)
-GLA(4)
-GLA(8)
+#define GLA(P) GLA_K(slm_gla_##P, P, false) GLA_K(slm_glah_##P, P, true)
 GLA(16)
+GLA(32)
+GLA(64)
+GLA(128)
+GLA(256)
 
 // ---------------------------------------------------------------------------------------
 // linear: y[i][r] = Σ_c w[r][c]·x[i][c] (ops.rs:116-126)
@@ -1197,12 +1211,6 @@ KERNEL void __launch_bounds__(256) slm_gemm(float* __restrict__ y, float* __rest
 // in order within the split, one split per blockIdx.z.
 #define GEMM_STAGES 2
 __device__ __forceinline__ int gsw(int row, int chunk) { return row * 64 + 4 * (chunk ^ (row & 15)); }
-
-template <int N>
-__device__ __forceinline__ void vm_wait() {  // s_waitcnt vmcnt(N), other counters untouched
-    static_assert(N >= 0 && N < 64, "vmcnt");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
 
 // The attention-input epilogue (ROPE, BM = dh = 64, rows = 3·d): y [m][3d] is written as
 // usual, and tile r0 is one head of q, k or v: q and k are also written rotated (slm_rope's
@@ -1676,35 +1684,6 @@ GEMM2(128, 16)
 // one workgroup, one wave per segment), superblocks into the result (slm_attn_combine).
 // Scores use the same 16x16x4 MFMA chain over dh as linear; P·V runs four MFMAs per tile
 // (MFMA r takes keys r, r+4, r+8, r+12).
-
-// v combined with lane l ^ 16 (or l ^ 32) through register lane swaps: v_permlane16_swap
-// gives every lane its row pair's even-row and odd-row values (v_permlane32_swap its half
-// pair's), so a symmetric op of the two is the lane's value with its partner's — the same bits
-// as op(v, shfl_xor(v, 16)) for the commutative max, + and |.
-__device__ __forceinline__ float xmax16(float v) {
-    auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
-}
-__device__ __forceinline__ float xmax32(float v) {
-    auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
-}
-__device__ __forceinline__ float xsum16(float v) {
-    auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
-}
-__device__ __forceinline__ float xsum32(float v) {
-    auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
-}
-__device__ __forceinline__ int xor16i(int v) {
-    auto p = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
-    return (int)(p[0] | p[1]);
-}
-__device__ __forceinline__ int xor32i(int v) {
-    auto p = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
-    return (int)(p[0] | p[1]);
-}
 
 // (M, L, O) ⊕= (mB, lB, oB); an empty partial (l = 0) changes nothing.
 __device__ __forceinline__ void fold(float& M, float& L, float& O, float mB, float lB,
@@ -3330,9 +3309,6 @@ __device__ __forceinline__ long long fg_row(const FgSeg& s, int t, int i) {
     return fg_row_of(s.rpt, s.pair_rows, s.half, s.mhalf, s.rows, t, i);
 }
 
-// Sixteen zero bytes: what a lane past the end of a weight matrix loads.
-__device__ __attribute__((aligned(16))) float slm_zero16[4];
-
 // Where one GEMV lane's weights of unit u come from, worked out once per unit: the
 // lane's row start (or the zero page), the first 16-column block of its slice and how
 // many of the slice's four blocks lie inside the matrix (0: the slice is past the end).
@@ -3906,8 +3882,8 @@ __device__ __forceinline__ bool gla1_body(const GlaDesc& g, int h, int tid, int 
     }
     // The state: where dh = 64 (RPL = 4, 1024 threads), thread t loads elements t, t + 1024, ...
     // (whole rows a wave, one memory line per 32 lanes) and the values reach their lanes
-    // through LDS (row a at a·65: lanes of one column read distinct banks); otherwise each
-    // lane loads its own rows of its column.
+    // through LDS (row a at a·68: a wave's sixteen rows of four columns fall on distinct banks);
+    // otherwise each lane loads its own rows (j, j + 16, ..) of its column.
     constexpr bool ST64 = RPL == 4;
     bool staged = ST64 && dh == 64 && nt == 1024;
     float* ls = lds + 4 * dh + 16;
@@ -3918,7 +3894,7 @@ __device__ __forceinline__ bool gla1_body(const GlaDesc& g, int h, int tid, int 
     } else {
 #pragma unroll
         for (int rr = 0; rr < RPL; rr++) {
-            int a = min(j * RPL + rr, dh - 1);
+            int a = min(j + 16 * rr, dh - 1);
             st[rr] = Sh[(long long)a * dh + bq];
         }
     }
@@ -3934,7 +3910,7 @@ __device__ __forceinline__ bool gla1_body(const GlaDesc& g, int h, int tid, int 
     if (!staged) {
 #pragma unroll
         for (int rr = 0; rr < RPL; rr++)
-            if (!live || j * RPL + rr >= dh) st[rr] = 0.0f;
+            if (!live || j + 16 * rr >= dh) st[rr] = 0.0f;
     }
     auto bar = [] {
         if (STEP) __syncthreads();
@@ -3978,11 +3954,11 @@ __device__ __forceinline__ bool gla1_body(const GlaDesc& g, int h, int tid, int 
 #pragma unroll
         for (int q = 0; q < RPL; q++) {
             int e = tid + q * 1024;
-            ls[(e >> 6) * 65 + (e & 63)] = st[q];
+            ls[(e >> 6) * 68 + (e & 63)] = st[q];
         }
         bar();
 #pragma unroll
-        for (int rr = 0; rr < RPL; rr++) st[rr] = ls[(j * RPL + rr) * 65 + b];
+        for (int rr = 0; rr < RPL; rr++) st[rr] = ls[(j + 16 * rr) * 68 + b];
     }
     bool hm = g.r16 != 0;
     float dc = hm ? gla_decay<true>(draw, bias) : gla_decay<false>(draw, bias);
@@ -3991,11 +3967,11 @@ __device__ __forceinline__ bool gla1_body(const GlaDesc& g, int h, int tid, int 
     if (hm) t2 = r16(t2);
     if (staged) {  // back through LDS (each lane's own slots), then whole rows a wave
 #pragma unroll
-        for (int rr = 0; rr < RPL; rr++) ls[(j * RPL + rr) * 65 + b] = st[rr];
+        for (int rr = 0; rr < RPL; rr++) ls[(j + 16 * rr) * 68 + b] = st[rr];
     } else {
 #pragma unroll
         for (int rr = 0; rr < RPL; rr++) {
-            int a = j * RPL + rr;
+            int a = j + 16 * rr;
             if (live && a < dh) Sh[(long long)a * dh + b] = st[rr];
         }
     }
@@ -4006,7 +3982,7 @@ __device__ __forceinline__ bool gla1_body(const GlaDesc& g, int h, int tid, int 
 #pragma unroll
         for (int q = 0; q < RPL; q++) {
             int e = tid + q * 1024;
-            Sh[e] = ls[(e >> 6) * 65 + (e & 63)];
+            Sh[e] = ls[(e >> 6) * 68 + (e & 63)];
         }
     }
     if (!g.fuse) return true;

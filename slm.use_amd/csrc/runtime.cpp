@@ -131,7 +131,7 @@ struct Kernels {
     // fp16 mode over fp16 weights (allocated with slm_hip_alloc_half)
     hipFunction_t lin_small_hw, fghw, gemm2hw[4], gemm2hsw[4], gemm2hrw, gemm2hnw;
     hipFunction_t lin_small[2], lin_big[2];  // [vec]
-    hipFunction_t gla[5], gla1[3];           // rows per lane 1, 2, 4, .. (16 lanes per column)
+    hipFunction_t gla[5], gla1[3];           // head sizes to 16, 32, .. 256; one token: to 16, 32, 64
     hipFunction_t glah[5];                   // the prompt GLA in fp16 mode
     hipFunction_t attn[5];                   // dim tiles 1, 2, 4, 8, 16
     hipFunction_t attn_dec[3];               // one-token attention, dim tiles 1, 2, 4
@@ -847,12 +847,14 @@ int lower_one(slm_hip* c, const Op& o, std::vector<Rec>& out) {
                              p[2], p[3], (long long)n[0], (long long)n[1], (long long)n[2]));
             return SLM_OK;
         case OP_GLA: {  // p0 y, p1 s, p2 q, p3 k, p4 v, p5 decay, p6 bias; n0 m, n1 heads, n2 dh
-            // sixteen lanes per state column, SLM_GLA_COLS columns per workgroup
+            // a lane a state row (GlaShape in kernels.hip): 4 columns a workgroup, 16 or 8 for
+            // heads of up to 16 or 32
             int i = pow2_index((n[2] + 15) / 16, 4);
-            uint32_t shmem = (uint32_t)(2 * SLM_GLA_T * (2 * n[2] + SLM_GLA_COLS + 1) * 4);  // two token groups
+            int64_t P = (int64_t)16 << i, nc = P < 64 ? 4 * (64 / P) : 4, T = P > 64 ? 16 : 32;
+            int64_t stage = T * 2 * P + 256 * ((T * (nc + 1) + 255) / 256);
+            uint32_t shmem = (uint32_t)((4 * stage + 4 * nc * T) * 4);
             int vec = (n[2] % 4 == 0 && aligned16(p[2]) && aligned16(p[3]) && aligned16(p[4])) ? 4 : 1;
-            out.push_back(mk(c->fp16 ? k.glah[i] : k.gla[i], (uint32_t)n[1], (uint32_t)((n[2] + SLM_GLA_COLS - 1) / SLM_GLA_COLS), 1,
-                             16 * SLM_GLA_COLS, shmem,
+            out.push_back(mk(c->fp16 ? k.glah[i] : k.gla[i], (uint32_t)n[1], (uint32_t)((n[2] + nc - 1) / nc), 1, 256, shmem,
                              p[0], p[1], p[2], p[3], p[4], p[5], p[6], (int)n[0], (int)n[1],
                              (int)n[2], vec));
             return SLM_OK;
@@ -2059,8 +2061,8 @@ struct Planner {
             }
         }
         int ri = pow2_index((dh + 15) / 16, 2);
-        // (dh = 64: the state staged in LDS, 64 rows of 65)
-        size_t stage = dh == 64 ? 64 * 65 : 0;
+        // (dh = 64: the state staged in LDS, 64 rows of 68)
+        size_t stage = dh == 64 ? 64 * 68 : 0;
         out.push_back(mk_desc(c->k.gla1[ri], (uint32_t)heads, (uint32_t)((dh * 16 + 63) / 64 * 64),
                               (uint32_t)((4 * dh + 16 + stage) * 4), d));
         return used;
@@ -3266,10 +3268,10 @@ int load_kernels(slm_hip* c) {
                {&k.lin_small_h, "slm_linear_small_vh"}, {&k.fgh, "slm_fgh"},
                {&k.lin_small[0], "slm_linear_small_s"}, {&k.lin_small[1], "slm_linear_small_v"},
                {&k.lin_big[0], "slm_linear_big_s"},     {&k.lin_big[1], "slm_linear_big_v"},
-               {&k.gla[0], "slm_gla_1"},   {&k.gla[1], "slm_gla_2"},   {&k.gla[2], "slm_gla_4"},
-               {&k.gla[3], "slm_gla_8"},   {&k.gla[4], "slm_gla_16"},
-               {&k.glah[0], "slm_glah_1"}, {&k.glah[1], "slm_glah_2"}, {&k.glah[2], "slm_glah_4"},
-               {&k.glah[3], "slm_glah_8"}, {&k.glah[4], "slm_glah_16"},
+               {&k.gla[0], "slm_gla_16"},   {&k.gla[1], "slm_gla_32"},   {&k.gla[2], "slm_gla_64"},
+               {&k.gla[3], "slm_gla_128"},   {&k.gla[4], "slm_gla_256"},
+               {&k.glah[0], "slm_glah_16"}, {&k.glah[1], "slm_glah_32"}, {&k.glah[2], "slm_glah_64"},
+               {&k.glah[3], "slm_glah_128"}, {&k.glah[4], "slm_glah_256"},
                {&k.gla1[0], "slm_gla1_1"}, {&k.gla1[1], "slm_gla1_2"}, {&k.gla1[2], "slm_gla1_4"},
                {&k.attn[0], "slm_attn_part_1"}, {&k.attn[1], "slm_attn_part_2"},
                {&k.attn[2], "slm_attn_part_4"}, {&k.attn[3], "slm_attn_part_8"},

@@ -1,0 +1,63 @@
+"""Kernels at the sizes where their tiling turns: one token more or less than a block or a
+stage, head sizes around the padded ones, the first and last sizes of a dispatch's ranges.
+References are the oracle or float64; every multi-token result is also compared bit for bit
+with the same tokens taken one at a time or a few at a time.
+"""
+
+import numpy as np
+import pytest
+
+import oracle as O
+from helpers import rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip(pkg):
+    h = pkg.Hip(0)
+    yield h
+    h.close()
+
+
+# blocks of 16 tokens in stages of 32 (head sizes to 64) or 16 (above), a ring of four stages;
+# heads padded to 16, 32, 64, 128 or 256 rows
+@pytest.mark.parametrize("fp16", [False, True])
+@pytest.mark.parametrize("m,heads,dh", [(15, 2, 64), (16, 2, 64), (17, 3, 64), (31, 1, 64), (33, 2, 64),
+                                        (128, 2, 64), (161, 2, 64), (49, 2, 60), (47, 2, 33), (63, 3, 17),
+                                        (16, 2, 16), (95, 1, 1), (34, 2, 65), (97, 1, 100), (15, 1, 129),
+                                        (81, 1, 200), (65, 1, 256)])
+def test_gla_blocks(hip, m, heads, dh, fp16):
+    """Against the oracle (2e-6, the bound of test_gpu_ops.py; fp16 mode rounds every element
+    and is compared with itself only), and the same bits one token at a time and in two calls."""
+    rng = np.random.default_rng(m * 1000 + dh)
+
+    def rnd(*shape, scale=1.0):
+        return (rng.standard_normal(shape) * scale).astype(np.float32)
+
+    q, k, v = rnd(m, heads, dh), rnd(m, heads, dh), rnd(m, heads, dh)
+    q /= np.linalg.norm(q, axis=-1, keepdims=True)
+    k /= np.linalg.norm(k, axis=-1, keepdims=True)
+    dec, bias, s0 = rnd(m, heads), rnd(heads) - 3, rnd(heads, dh, dh, scale=0.1)
+    hip.set_fp16(fp16)
+    try:
+        dq, dk, dv, dd, db = [hip.upload(t) for t in (q, k, v, dec, bias)]
+
+        def run(cuts):
+            ds, out = hip.upload(s0), []
+            for a, b in zip(cuts, cuts[1:]):
+                dy = hip.alloc((b - a) * heads * dh)
+                hip.gla(dy.ptr, ds.ptr, dq.at(a * heads * dh), dk.at(a * heads * dh), dv.at(a * heads * dh),
+                        dd.at(a * heads), db.ptr, b - a, heads, dh)
+                out.append(dy.read())
+            return np.concatenate(out), ds.read()
+
+        y, s = run([0, m])
+        for cuts in (list(range(m + 1)), [0, m // 3, m]):
+            y2, s2 = run([c for i, c in enumerate(cuts) if i == 0 or c > cuts[i - 1]])
+            assert np.array_equal(y, y2) and np.array_equal(s, s2)
+        if not fp16:
+            wy, ws = O.gla(s0, q, k, v, dec, bias, m, heads, dh)
+            assert rel(y, wy) < 2e-6 and rel(s, ws) < 2e-6
+    finally:
+        hip.set_fp16(False)
