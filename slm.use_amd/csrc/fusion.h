@@ -27,6 +27,8 @@
 #define SLM_FG_EPI_WAVES 4     // prologue/epilogue waves of slm_fg
 #define SLM_SB_SEGS 4          // 64-key attention segments per superblock
 #define SLM_SB_KEYS (64 * SLM_SB_SEGS)
+#define SLM_ATTN_QT 4         // query tiles (waves) per workgroup of the prompt attention
+#define SLM_ATTN_NB 2         // its LDS buffers of one 16-key tile each
 #define SLM_FG_MISC (32 + 4 * SLM_PF_MAX)  // LDS floats of slm_fg's scalars and prefetch table
 #define SLM_SIG_OPS 7          // prologue ops a signature can name
 // The signature of a prologue of kinds k0, k1, ...: what FgDesc.sig holds.

@@ -2000,18 +2000,20 @@ ATTN_PART(4)
 ATTN_PART(8)
 ATTN_PART(16)
 
-// Prompt attention with the keys and values of a superblock shared in LDS: a workgroup of
-// 16 waves takes ATTN_QG query tiles of one key head against one superblock. The waves
-// first copy the superblock's keys and values into LDS (rows of 16 chunks of 16 bytes, chunk
-// c at c ^ (key & 15)) — only the 16-key tiles some query of the workgroup sees, and nothing
-// at all for a superblock none sees (its partials are written empty); then wave w runs
-// segment w % 4 for query tile w / 4 with the arithmetic of attn_segment (operands from LDS
-// instead of registers; dims at or past dh read as zero, as there). The segments of each tile
-// are folded in order into superblock partials part[z][qidx][head][2 + 16·DT], which
+// Prompt attention: a workgroup of SLM_ATTN_QT waves takes as many query tiles of one key head
+// against one superblock, a tile a wave. The superblock's 16-key tiles of keys and values (rows
+// of 16 chunks of 16 bytes, chunk c at c ^ (key & 15)) pass through a ring of SLM_ATTN_NB LDS
+// buffers, the next tiles' copies in flight while one is used; only the tiles some query of
+// the workgroup sees are copied, and a superblock none sees is left out. A wave runs its query
+// tile over the tiles in order with the arithmetic of attn_segment and folds each segment's
+// partial into the superblock's in registers: part[z][qidx][head][2 + 16·DT], which
 // slm_attn_combine then combines. Grid (query tile groups, key heads, superblock slots),
 // placed XCD-aware (pq_place).
-#define ATTN_QG 4
-
+// Bound by issue (MFMAs and the softmax's vector instructions take turns on a SIMD): four such
+// workgroups of four waves share a CU, so one's copies and waits pass behind the others' tiles;
+// with all of a superblock staged at once (128 KB, one workgroup of 16 waves a CU) nothing
+// covered its copies and its fold. 256 queries, 12 heads of 64, a 4096-key window: 79.3 ->
+// 55.7 us a call with the combine (2 waves and 2 buffers 73.9, 4 and 3 56.4, 4 and 4 62.8).
 // Output dim of o[dt][r] in lane (i, g) of a prompt-attention wave. With DT = 4 the P·V MFMA
 // of block dt takes dims 4i + dt (A row i), so that the four values a lane needs of one key
 // are one 16-byte chunk (one LDS read per key instead of four); the accumulator then holds
@@ -2022,50 +2024,48 @@ __device__ __forceinline__ int pq_dim(int dt, int r, int g) {
     return DT == 4 ? 4 * (4 * g + r) + dt : 16 * dt + 4 * g + r;
 }
 
-// One 16-key tile (keys 16·st .. 16·st + 15 of the segment whose rows start at kt / vt) for
-// the wave's 16 columns; b0 is its first position; koff / voff are the lane's LDS offsets
-// (floats) of its key chunks (t) and value rows (r) in tile 0. FULL: dh = 16·DT (no dim
+// One 16-key tile, its rows at kt / vt, for the wave's 16 columns; b0 is its first key and
+// [lo_k, hi_k) the keys the lane's column sees, counted in the superblock;
+// kat / vat are the lane's byte offsets of key chunk 0 and value row 0 (chunk t and row r are
+// an exclusive or away, the swizzle being one). FULL: dh = 16·DT (no dim
 // tests). A tile that every valid column sees whole takes no per-key test (the same values:
 // a valid column's keys all pass, an invalid column's none); when every column is valid too,
 // every lane's state updates. A rescale by α = 1 (the running maximum unchanged in every
 // lane) is skipped: o·1 = o.
 template <int DT, bool FULL>
-__device__ __forceinline__ void pq_tile(const Col& col, bool allvalid, const f4 (&qv)[DT],
-                                        const float* kt, const float* vt, const int (&koff)[DT],
-                                        const int (&voff)[4], int st, long long b0, int dh,
+__device__ __forceinline__ void pq_tile(bool valid, int lo_k, int hi_k, bool allvalid, const f4 (&qv)[DT],
+                                        const char* kt, const char* vt, int kat, int vat, int b0, int dh,
                                         float scale, float& mo, float& lo, f4 (&o)[DT]) {
     int lane = threadIdx.x & 63;
     int i = lane & 15, g = lane >> 4;
-    bool sees = col.valid && col.lo < b0 + 16 && col.hi > b0;
+    bool sees = valid && lo_k < b0 + 16 && hi_k > b0;
     if (__ballot(sees) == 0) return;
-    bool whole = __ballot(col.valid && (col.lo > b0 || col.hi < b0 + 16)) == 0;
-    const float* kst = kt + 1024 * st;
-    const float* vst = vt + 1024 * st;
-    // scores' A operand: key 16st + i of the segment, dims 16t + 4g .. +3
+    bool whole = __ballot(valid && (lo_k > b0 || hi_k < b0 + 16)) == 0;
+    // scores' A operand: key i of the tile, dims 16t + 4g .. +3
     f4 kr[DT];
 #pragma unroll
     for (int t = 0; t < DT; t++) {
         kr[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (FULL || 16 * t + 4 * g < dh) kr[t] = *(const f4*)(kst + koff[t]);
+        if (FULL || 16 * t + 4 * g < dh) kr[t] = *(const f4*)(kt + (kat ^ (t << 6)));
     }
-    // values: MFMA r of block dt takes value of key 16st + 4g + r, dim pq_dim's A row i
+    // values: MFMA r of block dt takes value of key 4g + r, dim pq_dim's A row i
     float vr[4][DT];
     if (DT == 4) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             f4 w = f4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (FULL || 4 * i < dh) w = *(const f4*)(vst + voff[r]);
+            if (FULL || 4 * i < dh) w = *(const f4*)(vt + (vat ^ (r << 4)) + 256 * r);
 #pragma unroll
             for (int dt = 0; dt < DT; dt++) vr[r][dt] = w[dt];
         }
     } else {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            int kv = 16 * st + 4 * g + r;
+            int kv = 4 * g + r;
 #pragma unroll
             for (int dt = 0; dt < DT; dt++) {
                 int dd = 16 * dt + i;
-                vr[r][dt] = (FULL || dd < dh) ? vt[4 * (16 * kv + ((dd >> 2) ^ (kv & 15))) + (dd & 3)] : 0.0f;
+                vr[r][dt] = (FULL || dd < dh) ? ((const float*)vt)[4 * (16 * kv + ((dd >> 2) ^ kv)) + (dd & 3)] : 0.0f;
             }
         }
     }
@@ -2081,14 +2081,14 @@ __device__ __forceinline__ void pq_tile(const Col& col, bool allvalid, const f4 
     int anyi;
     if (whole) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) sv[r] = col.valid ? s[r] * scale : NEG_INF;
-        anyi = col.valid ? 1 : 0;
+        for (int r = 0; r < 4; r++) sv[r] = valid ? s[r] * scale : NEG_INF;
+        anyi = valid ? 1 : 0;
     } else {
         bool any = false;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            long long kp = b0 + 4 * g + r;
-            bool ok = kp >= col.lo && kp < col.hi;
+            int kp = b0 + 4 * g + r;
+            bool ok = kp >= lo_k && kp < hi_k;
             sv[r] = ok ? s[r] * scale : NEG_INF;
             any = any || ok;
         }
@@ -2121,18 +2121,18 @@ __device__ __forceinline__ void pq_tile(const Col& col, bool allvalid, const f4 
         mo = mnew;
         return;
     }
-    f4 on[DT];
+    // (a block at a time: one accumulator beside the state)
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++) on[dt] = o[dt] * alpha;
+    for (int dt = 0; dt < DT; dt++) {
+        f4 on = o[dt] * alpha;
 #pragma unroll
-    for (int r = 0; r < 4; r++)
+        for (int r = 0; r < 4; r++) on = mfma4(vr[r][dt], p[r], on);
 #pragma unroll
-        for (int dt = 0; dt < DT; dt++) on[dt] = mfma4(vr[r][dt], p[r], on[dt]);
+        for (int r = 0; r < 4; r++) o[dt][r] = anyi ? on[r] : o[dt][r];
+    }
     if (anyi) {
         lo = lo * alpha + rs;
         mo = mnew;
-#pragma unroll
-        for (int dt = 0; dt < DT; dt++) o[dt] = on[dt];
     }
 }
 
@@ -2157,30 +2157,20 @@ __device__ __forceinline__ void pq_place(int& gx, int& kvh, int& z) {
     z = (int)(unit / Y);
 }
 
-// The 16-key tiles [ta, tb) of a segment starting at position sbase that meet [LO, HI).
-__device__ __forceinline__ void pq_tiles(long long sbase, long long LO, long long HI, int& ta, int& tb) {
-    long long a = LO <= sbase ? 0 : (LO - sbase) >> 4;
-    long long b = HI <= sbase ? 0 : (HI - sbase + 15) >> 4;
-    tb = (int)(b < 4 ? b : 4);
-    ta = (int)(a < tb ? a : tb);
-}
-
 // With KH the rings hold fp16 values: the copies go through registers (four halves a lane,
 // widened exactly, written where the fp32 copy puts them); the rest is unchanged.
 template <int DT, bool FULL, bool KH = false>
-__device__ void attn_pq_run(float* __restrict__ part, const float* __restrict__ q,
+__device__ __forceinline__ void attn_pq_run(float* __restrict__ part, const float* __restrict__ q,
                             const float* __restrict__ kc, const float* __restrict__ vc,
                             long long pos, int m, long long reach, long long gap, long long cap,
                             int heads, int key_heads, int dh, float scale) {
     constexpr int DP = 16 * DT;
-    constexpr int NT = 64 * SLM_SB_SEGS * ATTN_QG;
-    constexpr int NC = ATTN_QG * 16;  // columns of the workgroup
-    extern __shared__ __attribute__((aligned(16))) float lds[];  // keys [256][64], values [256][64]; then the fold slots
-    float* kt = lds;
-    float* vt = lds + SLM_SB_KEYS * 64;
+    constexpr int NB = SLM_ATTN_NB, BUF = 2 * 16 * 64;  // floats of a tile's buffer: keys, then values
+    constexpr int NR = 4 / SLM_ATTN_QT;                 // row groups of four keys a wave copies of each
+    static_assert(SLM_ATTN_QT * NR == 4 && NB >= 2, "waves over a tile's copies");
+    extern __shared__ __attribute__((aligned(16))) float lds[];  // [NB][keys 16 x 64 | values 16 x 64], [waves][DT][64] f4
     int lane = threadIdx.x & 63;
     int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int seg = wave % SLM_SB_SEGS, qt = wave / SLM_SB_SEGS;
     int i = lane & 15, g = lane >> 4;
     int group = heads / key_heads, qpt = 16 / group;
     int gx, kvh, z;
@@ -2188,14 +2178,14 @@ __device__ void attn_pq_run(float* __restrict__ part, const float* __restrict__ 
     long long first = (reach - 1 > pos) ? 0 : pos - (reach - 1);
     long long k0 = (first / SLM_SB_KEYS + z) * SLM_SB_KEYS;  // the superblock's first position
     // every position some query of the workgroup sees lies in [LO, HI)
-    long long q0 = (long long)gx * ATTN_QG * qpt;
-    long long q1 = ((long long)m < q0 + ATTN_QG * qpt ? (long long)m : q0 + ATTN_QG * qpt) - 1;
+    long long q0 = (long long)gx * SLM_ATTN_QT * qpt;
+    long long q1 = ((long long)m < q0 + SLM_ATTN_QT * qpt ? (long long)m : q0 + SLM_ATTN_QT * qpt) - 1;
     long long LO = (reach - 1 > pos + q0) ? 0 : pos + q0 - (reach - 1);
     long long HI = (gap > pos + q1 + 1) ? 0 : pos + q1 + 1 - gap;
     // a superblock no query of the workgroup sees: nothing to write (slm_attn_combine reads
     // only the superblocks each row sees)
     if (HI <= LO || HI <= k0 || LO >= k0 + SLM_SB_KEYS) return;
-    Col col = column(i, (long long)gx * ATTN_QG + qt, pos, m, reach, gap, group, qpt, kvh);
+    Col col = column(i, (long long)gx * SLM_ATTN_QT + wave, pos, m, reach, gap, group, qpt, kvh);
     // this lane's share of its column's query: B[k = g][j = i] for each 16-dim block
     f4 qv[DT];
     const float* qrow = q + (col.qidx * heads + col.head) * (long long)dh;
@@ -2205,146 +2195,142 @@ __device__ void attn_pq_run(float* __restrict__ part, const float* __restrict__ 
         qv[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
         if (col.valid && (FULL || c < dh)) qv[t] = *(const f4*)(qrow + c);
     }
-    // the copies: wave w takes segment w / 4, and of each tile it copies the four keys
-    // 4·(w % 4) .. +3 (one instruction, lane L: key + L/16, chunk (L % 16) ^ (key & 15); a
-    // chunk at or past dh copies the row's last one, read as zero below)
-    h4 hk[KH ? 4 : 1], hv[KH ? 4 : 1];
-    int cs = wave >> 2, cta, ctb;
-    pq_tiles(k0 + 64 * cs, LO, HI, cta, ctb);
-    {
-        int nch = dh >> 2;
-        unsigned cap32 = (unsigned)cap;
-        unsigned base = (k0 >> 32) == 0 ? (unsigned)k0 % cap32 : (unsigned)(k0 % cap);
-        bool wrap1 = cap >= SLM_SB_KEYS;  // base + key < 2·cap: one subtraction wraps it
-        auto where = [&](int st, int& row) {  // the element offset of this lane's chunk of tile st
-            row = 64 * cs + 16 * st + 4 * (wave & 3);
-            int key = row + (lane >> 4);
-            int chunk = (lane & 15) ^ (key & 15);
-            if (!FULL || DT < 4) chunk = min(chunk, nch - 1);  // rows hold 16 chunks
-            unsigned slot = base + (unsigned)key;
-            slot = wrap1 ? (slot >= cap32 ? slot - cap32 : slot) : slot % cap32;
-            return (long long)slot * dh + 4 * chunk;
-        };
-        if constexpr (KH) {
-            const _Float16* kb = (const _Float16*)kc + (long long)kvh * cap * dh;
-            const _Float16* vb = (const _Float16*)vc + (long long)kvh * cap * dh;
+    // the superblock's tiles some query of the workgroup sees
+    constexpr int TILES = SLM_SB_KEYS / 16;
+    int ta = LO <= k0 ? 0 : (int)((LO - k0) >> 4);
+    long long tbl = (HI - k0 + 15) >> 4;
+    int tb = tbl < TILES ? (int)tbl : TILES;
+    // Copies of a tile: row group n (keys 4n .. 4n + 3) is one instruction for the keys and one
+    // for the values, lane L: key 4n + L/16, chunk (L % 16) ^ (key & 15); a chunk at or past
+    // dh copies the row's last one, read as zero below.
+    unsigned cap32 = (unsigned)cap;
+    unsigned base = (k0 >> 32) == 0 ? (unsigned)k0 % cap32 : (unsigned)(k0 % cap);
+    bool wrap1 = cap >= SLM_SB_KEYS;  // base + key < 2·cap: one subtraction wraps it
+    int chunk[NR];
 #pragma unroll
-            for (int st = 0; st < 4; st++) {
-                if (st < cta || st >= ctb) continue;
-                int row;
-                long long off = where(st, row);
-                hk[st] = gld((const h4*)(kb + off));
-                hv[st] = gld((const h4*)(vb + off));
-            }
-        } else {
-            const float* kb = kc + (long long)kvh * cap * dh;
-            const float* vb = vc + (long long)kvh * cap * dh;
-            for (int st = cta; st < ctb; st++) {
-                int row;
-                long long off = where(st, row);
+    for (int n = 0; n < NR; n++) {
+        chunk[n] = (lane & 15) ^ (4 * (wave + SLM_ATTN_QT * n) + g);
+        if (!FULL || DT < 4) chunk[n] = min(chunk[n], (dh >> 2) - 1);  // rows hold 16 chunks
+    }
+    auto where = [&](int t, int n) {
+        unsigned slot = base + (unsigned)(16 * t + 4 * (wave + SLM_ATTN_QT * n) + g);
+        if (wrap1) slot = slot >= cap32 ? slot - cap32 : slot;
+        else
+            while (slot >= cap32) slot -= cap32;
+        return (long long)slot * dh + 4 * chunk[n];
+    };
+    const float *kb = kc + (long long)kvh * cap * dh, *vb = vc + (long long)kvh * cap * dh;
+    const _Float16 *kh = (const _Float16*)kc + (long long)kvh * cap * dh, *vh = (const _Float16*)vc + (long long)kvh * cap * dh;
+    h4 hk[NR], hv[NR];  // (KH: the next tile's rows on their way)
+    auto issue = [&](int t) {
+#pragma unroll
+        for (int n = 0; n < NR; n++) {
+            long long off = where(t, n);
+            if constexpr (KH) {
+                hk[n] = gld((const h4*)(kh + off));
+                hv[n] = gld((const h4*)(vh + off));
+            } else {
+                float* dst = lds + (unsigned)t % NB * BUF + 256 * (wave + SLM_ATTN_QT * n);
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kb + off),
-                                                 (__attribute__((address_space(3))) void*)(kt + 64 * row), 16, 0, 0);
+                                                 (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vb + off),
-                                                 (__attribute__((address_space(3))) void*)(vt + 64 * row), 16, 0, 0);
+                                                 (__attribute__((address_space(3))) void*)(dst + 1024), 16, 0, 0);
             }
         }
-    }
-    bool allvalid = __ballot(col.valid) == ~0ull;
-    int koff[DT], voff[4];
+    };
+    auto widen = [&](int t) {  // (KH) the halves where the fp32 copies put their rows
 #pragma unroll
-    for (int t = 0; t < DT; t++) koff[t] = 64 * i + 4 * ((4 * t + g) ^ i);
-#pragma unroll
-    for (int r = 0; r < 4; r++) voff[r] = 64 * (4 * g + r) + 4 * (i ^ (4 * g + r));
-    vm_wait<0>();
-    if constexpr (KH) {  // the widened halves where the fp32 copies put their rows
-#pragma unroll
-        for (int st = 0; st < 4; st++) {
-            if (st < cta || st >= ctb) continue;
-            int row = 64 * cs + 16 * st + 4 * (wave & 3);
-            *(f4*)(kt + 64 * row + 4 * lane) = wide4(hk[st]);
-            *(f4*)(vt + 64 * row + 4 * lane) = wide4(hv[st]);
+        for (int n = 0; n < NR; n++) {
+            float* dst = lds + (unsigned)t % NB * BUF + 256 * (wave + SLM_ATTN_QT * n) + 4 * lane;
+            *(f4*)dst = wide4(hk[n]);
+            *(f4*)(dst + 1024) = wide4(hv[n]);
         }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    float mo = NEG_INF, lo = 0.0f;
+    };
+    constexpr int AHEAD = KH ? 1 : NB - 1;  // tiles in flight
+#pragma unroll
+    for (int p = 0; p < AHEAD; p++)
+        if (ta + p < tb) issue(ta + p);
+    // the keys the lane's column sees, counted from k0 (past the superblock: its end)
+    bool valid = col.valid, allvalid = __ballot(valid) == ~0ull;
+    int lo_k = col.lo <= k0 ? 0 : (int)(col.lo - k0 < SLM_SB_KEYS ? col.lo - k0 : SLM_SB_KEYS);
+    int hi_k = col.hi <= k0 ? 0 : (int)(col.hi - k0 < SLM_SB_KEYS ? col.hi - k0 : SLM_SB_KEYS);
+    float* P = part + (((long long)z * m + col.qidx) * heads + col.head) * (long long)(DP + 2);
+    int kat = 256 * i + 16 * (g ^ i), vat = 1024 * g + 16 * (i ^ (4 * g));
+    float FM = NEG_INF, FL = 0.0f, mo = NEG_INF, lo = 0.0f;
     f4 o[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) o[dt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    {
-        long long sbase = k0 + 64 * seg;
-        int ta, tb;
-        pq_tiles(sbase, LO, HI, ta, tb);
-        const float* ks = kt + seg * 64 * 64;
-        const float* vs = vt + seg * 64 * 64;
-#pragma unroll
-        for (int st = 0; st < 4; st++) {
-            if (st < ta || st >= tb) continue;
-            pq_tile<DT, FULL>(col, allvalid, qv, ks, vs, koff, voff, st, sbase + 16 * st, dh,
-                              scale, mo, lo, o);
+    // the superblock's o, in the wave's own LDS (touched once a segment: its registers are
+    // worth more to the tiles, four waves a SIMD being 128)
+    f4* FO = (f4*)(lds + NB * BUF) + wave * DT * 64 + lane;
+    if constexpr (KH) widen(ta);
+    for (int t = ta; t < tb; t++) {
+        // tile t is in (this wave's copies, then everyone's), and every wave is done with tile
+        // t − 1, whose buffer the next copies take
+        if constexpr (!KH) {
+            if (t + NB - 2 < tb) vm_wait<(NB - 2) * 2 * NR>();
+            else vm_wait<0>();
         }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (t + AHEAD < tb) issue(t + AHEAD);
+        const char* buf = (const char*)(lds + (unsigned)t % NB * BUF);
+        pq_tile<DT, FULL>(valid, lo_k, hi_k, allvalid, qv, buf, buf + 4096, kat, vat, 16 * t, dh, scale, mo, lo, o);
+        if constexpr (KH)
+            if (t + 1 < tb) widen(t + 1);
+        if ((t & 3) != 3 && t + 1 < tb) continue;
+        // the segment's end: its partial folds into the superblock's (fold()'s expressions; lanes
+        // of one column hold the same m and l)
+        if (__ballot(FL != 0.0f) == 0) {
+            FM = mo;
+            FL = lo;
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++) FO[64 * dt] = o[dt];
+        } else if (__ballot(lo != 0.0f) != 0) {
+            float mn = fmaxf(FM, mo);
+            float a = expf(FM - mn), b = expf(mo - mn);
+            bool none = lo == 0.0f, open = FL == 0.0f;
+            FL = none ? FL : open ? lo : FL * a + lo * b;
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++) {
+                f4 F = FO[64 * dt];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float v = F[r] * a + o[dt][r] * b;
+                    F[r] = none ? F[r] : open ? o[dt][r] : v;
+                }
+                FO[64 * dt] = F;
+            }
+            FM = none ? FM : mn;
+        }
+        mo = NEG_INF;
+        lo = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) o[dt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    __syncthreads();  // every wave is done with the keys and values: their LDS holds the folds
-    // fold each tile's segments in order (fold()'s expressions): wave (tile, s) takes the
-    // accumulator registers r = s of the tile's four segment waves, lane for lane (lane i of
-    // every one of them holds column i), with the column's (m, l) of each segment
-    f4* X = (f4*)lds;                                       // [wave][r][lane]: o[0..3][r]
-    float2* Y = (float2*)(lds + 4 * (SLM_SB_SEGS * ATTN_QG) * 4 * 64);  // [wave][lane]: (m, l)
+    if (!valid) return;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) o[dt] = FO[64 * dt];
+    if (g == 0) *(float2*)P = float2{FM, FL};
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-        f4 v = f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int dt = 0; dt < DT; dt++) v[dt] = o[dt][r];
-        X[(wave * 4 + r) * 64 + lane] = v;
-    }
-    Y[wave * 64 + lane] = float2{mo, lo};
-    __syncthreads();
-    // (with fewer than four segment waves a tile, each takes the registers r = s, s + SEGS, ..)
-    static_assert(4 % SLM_SB_SEGS == 0, "accumulator registers over the segment waves");
-#pragma unroll
-    for (int r = seg; r < 4; r += SLM_SB_SEGS) {
-        f4 xv[SLM_SB_SEGS];
-        float2 ml[SLM_SB_SEGS];
-#pragma unroll
-        for (int w = 0; w < SLM_SB_SEGS; w++) {
-            xv[w] = X[((qt * SLM_SB_SEGS + w) * 4 + r) * 64 + lane];
-            ml[w] = Y[(qt * SLM_SB_SEGS + w) * 64 + lane];
-        }
-        float FM = NEG_INF, FL = 0.0f;
-        f4 FO = f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int w = 0; w < SLM_SB_SEGS; w++) {
-            float mB = ml[w].x, lB = ml[w].y;
-            if (lB == 0.0f) continue;
-            if (FL == 0.0f) {
-                FM = mB;
-                FL = lB;
-                FO = xv[w];
-                continue;
+        if constexpr (DT == 4) {  // dims 16g + 4r + 0..3 (rows of DP + 2 floats: 8-byte aligned)
+            int dd = pq_dim<DT>(0, r, g);
+            if (FULL || dd < dh) {
+                *(float2*)(P + 2 + dd) = float2{o[0][r], o[1][r]};
+                *(float2*)(P + 4 + dd) = float2{o[2][r], o[3][r]};
             }
-            float mn = fmaxf(FM, mB);
-            float a = expf(FM - mn), b = expf(mB - mn);
-            FL = FL * a + lB * b;
-#pragma unroll
-            for (int dt = 0; dt < DT; dt++) FO[dt] = FO[dt] * a + xv[w][dt] * b;
-            FM = mn;
-        }
-        if (col.valid) {
-            float* P = part + (((long long)z * m + col.qidx) * heads + col.head) * (long long)(DP + 2);
-            if (g == 0 && r == 0) {
-                P[0] = FM;
-                P[1] = FL;
-            }
+        } else {
 #pragma unroll
             for (int dt = 0; dt < DT; dt++) {
                 int dd = pq_dim<DT>(dt, r, g);
-                if (FULL || dd < dh) P[2 + dd] = FO[dt];
+                if (FULL || dd < dh) P[2 + dd] = o[dt][r];
             }
         }
     }
 }
 
 #define ATTN_PQ(NAME, DT, KH)                                                            \
-    KERNEL void __launch_bounds__(64 * SLM_SB_SEGS * ATTN_QG) NAME(                       \
+    KERNEL void __launch_bounds__(64 * SLM_ATTN_QT, 4) NAME(                                  \
         float* part, const float* q, const float* kc, const float* vc,                   \
         const long long* dyn, long long pos_imm, int m, long long reach, long long gap,  \
         long long cap, int heads, int key_heads, int dh, float scale) {                  \

@@ -55,7 +55,6 @@ constexpr int LDS_MAX = 163840;            // gfx950: 160 KB of LDS per workgrou
 constexpr int FG_GRID_MAX = 256;           // workgroups of a fused GEMV: one per compute unit
 constexpr int64_t ATTN_CTR_MAX = 65536;   // (query tile, key head) pairs one attention launch combines itself
 constexpr int ATTN_LDS_MAX = LDS_MAX;
-constexpr int ATTN_QG_HOST = 4;   // query tiles per workgroup of the prompt attention (ATTN_QG)
 constexpr int ATTN_DEC_LDS = SLM_SB_SEGS * (2 * 64 * 64 + 1024) * 4;  // one-token attention: 256 keys and values, queries
 constexpr int GEMM_STAGES_HOST = 2;          // slices in flight in slm_gemm2 (GEMM_STAGES)
 constexpr int64_t CU_COUNT = 256;           // MI355X compute units
@@ -877,13 +876,13 @@ int lower_one(slm_hip* c, const Op& o, std::vector<Rec>& out) {
             if (attn_dec_ok(o)) return lower_attn_dec(c, o, out, false);
             float* part = attn_part(c, o);
             int64_t qpt = 16 / (heads / kh);
-            int64_t groups = ((m + qpt - 1) / qpt + ATTN_QG_HOST - 1) / ATTN_QG_HOST;
+            int64_t groups = ((m + qpt - 1) / qpt + SLM_ATTN_QT - 1) / SLM_ATTN_QT;
             if (m > 1 && dh <= 64 && groups * kh * nsb <= (int64_t)INT_MAX) {
-                // a superblock's keys and values shared in LDS by four query tiles
+                // a superblock's keys and values pass through LDS for SLM_ATTN_QT query tiles
                 // (then every row's superblocks are combined by a kernel of their own: many
                 // rows, each a wave, rather than one workgroup per tile group at the end)
                 out.push_back(mk(n[9] ? k.attn_pq16[dti] : k.attn_pq[dti], (uint32_t)groups, (uint32_t)kh, (uint32_t)nsb,
-                                 64 * SLM_SB_SEGS * ATTN_QG_HOST, (uint32_t)(2 * SLM_SB_KEYS * 64 * 4),
+                                 64 * SLM_ATTN_QT, (uint32_t)((SLM_ATTN_NB * 2 + SLM_ATTN_QT) * 16 * 64 * 4),
                                  part, p[1], p[2], p[3], (const long long*)o.dyn, (long long)n[0],
                                  (int)m, (long long)n[2], (long long)n[3], (long long)n[4],
                                  (int)heads, (int)kh, (int)dh, o.f[0]));
@@ -4306,7 +4305,7 @@ int attend_op(slm_hip* c, float* y, const float* q, const float* k, const float*
     o.n[8] = (int64_t)nsb;
     o.n[9] = hk ? 1 : 0;
     o.f[0] = c->fp16 ? round16(a->scale) : a->scale;  // (fp16 mode: the dtype's scalar, mlx.rs:344)
-    if (hk && m > 1 && (int64_t)((qtiles + ATTN_QG_HOST - 1) / ATTN_QG_HOST) * (int64_t)kh * (int64_t)nsb > (int64_t)INT_MAX)
+    if (hk && m > 1 && (int64_t)((qtiles + SLM_ATTN_QT - 1) / SLM_ATTN_QT) * (int64_t)kh * (int64_t)nsb > (int64_t)INT_MAX)
         return fail(c, SLM_E_UNSUPPORTED, "attend: fp16 rings: %zu query tiles", qtiles);
     return SLM_OK;
 }

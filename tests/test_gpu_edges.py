@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from helpers import rel
+from helpers import attend64, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +61,29 @@ def test_gla_blocks(hip, m, heads, dh, fp16):
             assert rel(y, wy) < 2e-6 and rel(s, ws) < 2e-6
     finally:
         hip.set_fp16(False)
+
+
+# four query tiles of 16 / group queries a workgroup; 16-key tiles, 64-key segments, 256-key
+# superblocks; rings shorter than a superblock, spans that start or end inside a tile
+@pytest.mark.parametrize("pos,m,reach,gap,cap,heads,kh,dh", [
+    (0, 2, O.USIZE_MAX, 0, 300, 2, 2, 64), (0, 64, O.USIZE_MAX, 0, 64, 1, 1, 64), (1000, 65, 100, 0, 165, 2, 2, 64),
+    (255, 17, 256, 0, 512, 1, 1, 64), (513, 63, 49, 0, 112, 2, 1, 60), (300, 33, O.USIZE_MAX, 64, 400, 8, 1, 64),
+    (77, 129, 15, 0, 144, 4, 2, 32), (2000, 16, 1024, 0, 1040, 3, 3, 16), (40, 100, 8, 0, 24 + 100, 2, 1, 4)])
+def test_attend_tiles(hip, pos, m, reach, gap, cap, heads, kh, dh):
+    """Against float64 (no further than twice the oracle's fp32 sums, as test_gpu_ops.py), and
+    every query alone gives the same bits; slots no query sees hold NaN."""
+    rng = np.random.default_rng(pos * 1000 + m)
+    a = dict(pos=pos, m=m, reach=reach, gap=gap, cap=cap, heads=heads, key_heads=kh, dh=dh,
+             scale=float(1 / np.sqrt(dh)))
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((m, heads, dh), (kh, cap, dh), (kh, cap, dh)))
+    first, last = max(0, pos - reach + 1), max(0, pos + m - gap)
+    unseen = sorted(set(range(cap)) - {p % cap for p in range(first // 16 * 16, (last + 15) // 16 * 16)})
+    k[:, unseen] = v[:, unseen] = np.nan
+    dq, dk, dv, dy, d1 = hip.upload(q), hip.upload(k), hip.upload(v), hip.alloc(q.size), hip.alloc(heads * dh)
+    hip.attend(dy.ptr, dq.ptr, dk.ptr, dv.ptr, **a)
+    got = dy.read().reshape(m, -1)
+    for i in range(m):
+        hip.attend(d1.ptr, dq.at(i * heads * dh), dk.ptr, dv.ptr, **dict(a, pos=pos + i, m=1))
+        assert np.array_equal(d1.read(), got[i]), i
+    want, exact = O.attend(q, k, v, **a), attend64(q, k, v, **a)
+    assert rel(got.ravel(), exact) <= 2 * rel(want, exact) + 1e-7
