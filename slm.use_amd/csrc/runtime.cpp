@@ -4304,7 +4304,8 @@ int attend_op(slm_hip* c, float* y, const float* q, const float* k, const float*
     o.n[7] = (int64_t)dh;
     o.n[8] = (int64_t)nsb;
     o.n[9] = hk ? 1 : 0;
-    o.f[0] = c->fp16 ? round16(a->scale) : a->scale;  // (fp16 mode: the dtype's scalar, mlx.rs:344)
+    // the kernels' scores are in powers of two (fp16 mode: the dtype's scalar first, mlx.rs:344)
+    o.f[0] = (float)((double)(c->fp16 ? round16(a->scale) : a->scale) * 1.4426950408889634);
     if (hk && m > 1 && (int64_t)((qtiles + SLM_ATTN_QT - 1) / SLM_ATTN_QT) * (int64_t)kh * (int64_t)nsb > (int64_t)INT_MAX)
         return fail(c, SLM_E_UNSUPPORTED, "attend: fp16 rings: %zu query tiles", qtiles);
     return SLM_OK;
