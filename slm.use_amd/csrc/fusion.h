@@ -59,6 +59,9 @@ enum {
                     // ((long long*)o1)[0] and ((unsigned*)o2)[slot] (o2 may be null; slot:
                     // dyn[0], else imm); o3: [0] the 64-bit key of the running maximum,
                     // [2] the count of finished workgroups (both zero between launches)
+    EPI_SCALE = 5,  // y; o1 = y · factor (dyn[0] as a float, else imm's low bits)
+    EPI_STORE = 6,  // y; rows d .. d + half into cache o3 [half/dh][cap][dh] at slot dyn[0] (else imm)
+                    // mod cap; o4 (may be null): the next `half` rows, slot dyn2[0] (else imm2)
 };
 
 // A global vector copied into LDS by the prologue waves: src + dyn[0]·stride (when dyn).

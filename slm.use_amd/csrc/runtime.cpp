@@ -964,6 +964,10 @@ bool vp_of(const Op& o, VpSrc* v) {
             if (n[0] != 1) return false;
             v->kind = SRC_SCALE; v->n = (int)n[1]; v->in[0] = o.p[1]; v->out[0] = o.p[0];
             break;
+        case OP_SHIFT:  // (one row: the kept row alone)
+            if (n[0] != 1) return false;
+            v->kind = SRC_COPY; v->n = (int)n[1]; v->in[0] = o.p[1]; v->out[0] = o.p[0];
+            break;
         case OP_GATHER:
             if (n[0] != 1) return false;
             v->kind = SRC_GATHER; v->n = (int)n[1]; v->out[0] = o.p[0];
@@ -1012,7 +1016,7 @@ void op_ranges(const Op& o, std::vector<Range>& rd, std::vector<Range>& wr) {
         case OP_SHIFT:
             wr.push_back(rng(p[0], n[0] * n[1]));
             rd.push_back(rng(p[1], n[1]));
-            rd.push_back(rng(p[2], n[0] * n[1]));
+            if (n[0] > 1) rd.push_back(rng(p[2], (n[0] - 1) * n[1]));
             break;
         case OP_COLUMNS: wr.push_back(rng(p[0], n[0] * n[3])); rd.push_back(rng(p[1], n[0] * n[1])); break;
         case OP_LINEAR:
@@ -1089,6 +1093,62 @@ bool dead_after(const std::vector<Op>& ops, size_t from, const Range& r) {
             if (x.a <= r.a && r.b <= x.b) return true;
     }
     return false;
+}
+
+// May ops a and b change places? (nothing one writes is read or written by the other)
+bool commute(const Op& a, const Op& b) {
+    std::vector<Range> ra, wa, rb, wb;
+    op_ranges(a, ra, wa);
+    op_ranges(b, rb, wb);
+    for (auto& w : wa) {
+        for (auto& x : rb)
+            if (overlap(w, x)) return false;
+        for (auto& x : wb)
+            if (overlap(w, x)) return false;
+    }
+    for (auto& w : wb)
+        for (auto& x : ra)
+            if (overlap(w, x)) return false;
+    return true;
+}
+
+// A global layer's one-token step (model.rs:486-528, with kshift): q and kv = linears of n, [q
+// scaled], shifted = the kept row, kv' = linear(shifted), the kept row = n, k into its cache
+// from kv', v from kv. The kept row is the last step's, so shifted, kv' and the store of k move
+// up to before the down projection of the block before, where nothing is pending (or before the
+// element-wise ops ahead of q): they become one fused GEMV that waits for nothing of this
+// block, and q, kv, the scale, the store of v and the kept row's copy another. Only where every
+// op passed reads and writes elsewhere.
+std::vector<Op> order_global(const std::vector<Op>& in) {
+    std::vector<Op> ops = in;
+    for (size_t t = 2; t + 4 < ops.size(); t++) {
+        const Op &sh = ops[t], &ln = ops[t + 1], &cp = ops[t + 2], &sk = ops[t + 3], &sv = ops[t + 4];
+        if (sh.kind != OP_SHIFT || sh.n[0] != 1 || ln.kind != OP_LINEAR || ln.n[2] != 1 || ln.p[2] != sh.p[0] ||
+            cp.kind != OP_COPY || sk.kind != OP_STORE || sv.kind != OP_STORE || sk.p[1] != ln.p[0])
+            continue;
+        if (!commute(cp, sk) || !commute(cp, sv) || !commute(sk, sv)) continue;
+        auto free_of = [&](size_t j) {
+            return commute(ops[j], sh) && commute(ops[j], ln) && commute(ops[j], sk);
+        };
+        size_t lo = t;  // the ops from lo on may all be passed
+        while (lo > 0 && t - lo < 16 && free_of(lo - 1)) lo--;
+        size_t at = t;
+        for (size_t j = t; j > lo; j--)
+            if (ops[j - 1].kind == OP_SILU_MUL) { at = j; break; }
+        if (at == t) {  // no MLP before: ahead of q's linears and their element-wise inputs
+            size_t j = t, lin = 0;
+            VpSrc v;
+            while (j > lo && (ops[j - 1].kind == OP_LINEAR ? ops[j - 1].n[2] == 1 && ++lin <= 2 : vp_of(ops[j - 1], &v))) j--;
+            if (lin) at = j;
+        }
+        std::vector<Op> mv = {sh, ln, sk}, rest(ops.begin() + at, ops.begin() + t);
+        rest.push_back(sv);
+        rest.push_back(cp);
+        std::copy(mv.begin(), mv.end(), ops.begin() + at);
+        std::copy(rest.begin(), rest.end(), ops.begin() + at + 3);
+        t += 4;
+    }
+    return ops;
 }
 
 // Builds one slm_fg launch: LDS slots, prefetches, prologue ops, segments.
@@ -1730,6 +1790,66 @@ struct Planner {
                 hold_k = &lk;
             }
         }
+        // a second matrix on the same input (a global layer's q and kv, model.rs:493-494)
+        bool pair = false;
+        if (s0.epi == EPI_PLAIN && nseg == 1 && nsplit == 1 && is(i + 1, OP_LINEAR)) {
+            const Op& D = ops[i + 1];
+            if (D.n[2] == 1 && D.p[2] == x && D.n[1] == cols && D.n[0] >= 1 && D.n[0] <= (int64_t)1 << 26 &&
+                aligned16(D.p[1]) && D.n[3] == L.n[3] && D.n[4] == L.n[4] &&
+                !overlap(rng(D.p[0], D.n[0]), rng(y, rows)) && !overlap(rng(x, cols), rng(y, rows))) {
+                seg_init(seg[1], D);
+                nseg = 2;
+                used = 2;
+                pair = true;
+            }
+        }
+        // a factor on a matrix's output; stores of parts of one into caches (model.rs:495-528)
+        auto seg_of = [&](const float* p, int64_t n) {
+            for (int k = 0; k < nseg; k++)
+                if (p >= seg[k].y && p + n <= seg[k].y + seg[k].rows) return k;
+            return -1;
+        };
+        bool plain = s0.epi == EPI_PLAIN && nsplit == 1 && !hold_q;
+        if (plain && is(i + used, OP_SCALE_ROWS) && ops[i + used].n[0] == 1) {
+            const Op& sc = ops[i + used];
+            int k = seg_of(sc.p[1], sc.n[1]);
+            if (k >= 0 && seg[k].epi == EPI_PLAIN && sc.p[1] == seg[k].y && sc.n[1] == seg[k].rows) {
+                seg[k].epi = EPI_SCALE;
+                seg[k].o1 = (float*)sc.p[0];
+                seg[k].dyn = (const long long*)sc.dyn;
+                uint32_t bits;
+                std::memcpy(&bits, &sc.f[0], 4);
+                seg[k].imm = bits;
+                used++;
+            }
+        }
+        while (plain && is(i + used, OP_STORE) && ops[i + used].n[0] == 1) {
+            const Op& st = ops[i + used];
+            int64_t len = st.n[2] * st.n[3];
+            int k = seg_of(st.p[1], len);
+            if (k < 0) break;
+            FgSeg& g = seg[k];
+            int64_t off = st.p[1] - g.y;
+            if (g.epi == EPI_PLAIN) {
+                g.epi = EPI_STORE;
+                g.d = (int32_t)off;
+                g.half = (int32_t)len;
+                g.dh = (int32_t)st.n[3];
+                g.cap = st.n[1];
+                g.ring16 = (int32_t)st.n[5];
+                g.o3 = (float*)st.p[0];
+                g.dyn = (const long long*)st.dyn;
+                g.imm = st.n[4];
+            } else if (g.epi == EPI_STORE && !g.o4 && off == g.d + g.half && len == g.half && st.n[3] == g.dh &&
+                       st.n[1] == g.cap && (int32_t)st.n[5] == g.ring16) {
+                g.o4 = (float*)st.p[0];
+                g.dyn2 = (const long long*)st.dyn;
+                g.imm2 = st.n[4];
+            } else {
+                break;
+            }
+            used++;
+        }
         // MLP up: SiLU of the gate half times the amp half (model.rs:552-555)
         if (s0.epi == EPI_PLAIN && nseg == 1 && nsplit == 1 && is(i + 1, OP_SILU_MUL)) {
             const Op& sm = ops[i + 1];
@@ -1772,9 +1892,14 @@ struct Planner {
         }
         int64_t nsl = (cols / 16 + SLM_KS - 1) / SLM_KS;
         int W = (int)std::min<int64_t>(nsl, SLM_SPLIT);
-        if (nseg == 1) {
-            s0.rpt = choose_rpt(s0, cols, L.n[4] ? 2.0 : 4.0, c->fg_rpt);
-            s0.tiles = (s0.rows + s0.rpt - 1) / s0.rpt;
+        if (nseg == 1 || pair) {
+            FgSeg both = s0;  // (two matrices: tiles for their rows together)
+            if (pair) both.rows += seg[1].rows;
+            int rpt = choose_rpt(both, cols, L.n[4] ? 2.0 : 4.0, c->fg_rpt);
+            for (int k = 0; k < nseg; k++) {
+                seg[k].rpt = rpt;
+                seg[k].tiles = (seg[k].rows + rpt - 1) / rpt;
+            }
         }
         // what the segments read and write
         int units = 0;
@@ -1792,6 +1917,11 @@ struct Planner {
             switch (s.epi) {
                 case EPI_RESID: b.writes.push_back(rng(s.o1, s.rows)); break;
                 case EPI_SILU: b.writes.push_back(rng(s.o1, s.half)); break;
+                case EPI_SCALE: b.writes.push_back(rng(s.o1, s.rows)); break;
+                case EPI_STORE:
+                    for (float* o : {s.o3, s.o4})
+                        if (o) b.writes.push_back(rng(o, ring_floats((int64_t)(s.half / s.dh) * s.cap * s.dh, s.ring16)));
+                    break;
                 case EPI_PICK: {
                     const Op& a = ops[i + 1];
                     b.writes.push_back(rng(a.p[0], 2));
@@ -1891,7 +2021,10 @@ struct Planner {
             for (int k = 0; k < b.d.nvp; k++) {
                 VpOp& o = b.d.vp[k];
                 if (!o.gout) continue;
-                if (dead_after(ops, i + used, rng(o.gout, o.n)))
+                Range g = rng(o.gout, o.n);
+                bool over = false;  // the epilogue writes all of it (after: the op came before the linear)
+                for (auto& w : b.writes) over = over || (!w.wg0 && w.a <= g.a && g.b <= w.b);
+                if (over || dead_after(ops, i + used, g))
                     o.gout = nullptr;
                 else
                     kept.push_back(rng0(o.gout, o.n));
@@ -2348,7 +2481,11 @@ struct Planner {
 
 int plan(slm_hip* c, const std::vector<Op>& ops, std::vector<Rec>& out, bool fuse,
          std::vector<PlanMark>* marks = nullptr) {
-    Planner p{c, ops, out, marks, {}};
+    bool shifts = false;
+    for (const Op& o : ops) shifts = shifts || (o.kind == OP_SHIFT && o.n[0] == 1);
+    std::vector<Op> moved;
+    if (fuse && shifts && !marks) moved = order_global(ops);
+    Planner p{c, moved.empty() ? ops : moved, out, marks, {}};
     size_t before = out.size();
     TRY(p.run(fuse));
     if (c->plan_trace) {

@@ -87,3 +87,60 @@ def test_attend_tiles(hip, pos, m, reach, gap, cap, heads, kh, dh):
         assert np.array_equal(d1.read(), got[i]), i
     want, exact = O.attend(q, k, v, **a), attend64(q, k, v, **a)
     assert rel(got.ravel(), exact) <= 2 * rel(want, exact) + 1e-7
+
+
+@pytest.mark.parametrize("fp16", [False, True])
+@pytest.mark.parametrize("d,kh,dh,cap,shift,logn", [(768, 4, 64, 300, True, True), (768, 4, 64, 128, False, True),
+                                                    (64, 1, 16, 64, True, False), (128, 2, 48, 65, False, False)])
+def test_global_layer_input(hip, d, kh, dh, cap, shift, logn, fp16):
+    """A global layer's one-token input (two matrices on one input, a scaled output, stores out
+    of parts of an output, the kept row's matrix moved ahead) leaves the bits of one launch per
+    operation in every buffer, in fewer kernels, step after step."""
+    rng = np.random.default_rng(d + cap)
+    hip.set_fp16(fp16)
+    try:
+        kd = kh * dh
+        up = lambda *s, scale=1.0: hip.upload((rng.standard_normal(s) * scale).astype(np.float32))  # noqa: E731
+        inv = hip.upload(np.ones(8, np.float32))
+        cs, sn = hip.alloc(8), hip.alloc(8)
+        wq, wkv, wm, g = up(d, d, scale=0.05), up(2 * kd, d, scale=0.05), up(d, 2 * d, scale=0.05), up(d)
+        x, prev, up2 = up(d), up(d), up(4 * d)
+        bufs = dict(n=hip.alloc(d), q=hip.alloc(d), q2=hip.alloc(d), kv=hip.alloc(2 * kd), kv2=hip.alloc(2 * kd),
+                    sh=hip.alloc(d), t=hip.alloc(d), mid=hip.alloc(2 * d), h=hip.alloc(d), prev=prev,
+                    k=hip.alloc_cache(kh, cap, dh), v=hip.alloc_cache(kh, cap, dh))
+        b = {n: t.ptr for n, t in bufs.items()}
+        first = prev.read()
+
+        def step(pos, fuse):
+            hip.set_fusion(fuse)
+            hip.rope_table(cs.ptr, sn.ptr, inv.ptr, pos, 1, 8)
+            hip.silu_mul(b["mid"], up2.at(0), up2.at(2 * d), 2 * d)
+            hip.linear(b["h"], wm.ptr, d, 2 * d, b["mid"], 1)
+            hip.add(b["t"], x.ptr, b["h"], d)
+            hip.rms(b["n"], b["t"], g.ptr, 1, d, 1e-6)
+            hip.linear(b["q"], wq.ptr, d, d, b["n"], 1)
+            hip.linear(b["kv"], wkv.ptr, 2 * kd, d, b["n"], 1)
+            if logn:
+                hip.scale_rows(b["q2"], b["q"], np.array([0.37 + pos], np.float32), d)
+            if shift:
+                hip.shift(b["sh"], b["prev"], b["n"], 1, d)
+                hip.linear(b["kv2"], wkv.ptr, 2 * kd, d, b["sh"], 1)
+                hip.copy(b["prev"], b["n"], d)
+            hip.store(b["k"], b["kv2" if shift else "kv"], pos, 1, cap, kh, dh)
+            hip.store(b["v"], bufs["kv"].at(kd), pos, 1, cap, kh, dh)
+            hip.flush([t.ptr for t in bufs.values()])
+            return hip.last_plan()["kernels"]
+
+        got, kernels = {}, {}
+        for fuse in (False, True):
+            hip.upload_into(prev, first)
+            for t in ("k", "v"):
+                hip.upload_into(bufs[t], np.zeros(kh * cap * dh, np.float32))
+            kernels[fuse] = [step(pos, fuse) for pos in (3, 4, cap - 1, cap, 2 * cap + 7)]
+            got[fuse] = {n: t.read() for n, t in bufs.items()}
+        for n in got[False]:
+            assert np.array_equal(got[False][n], got[True][n]), n
+        assert max(kernels[True]) <= 5 < min(kernels[False])
+    finally:
+        hip.set_fusion(True)
+        hip.set_fp16(False)
