@@ -914,195 +914,17 @@ GLA(256)
 // + ..., and the split sums are added in order: y = ((Q0 + Q1) + Q2) + ...  Columns past
 // `cols` load as zero.
 
-template <bool VEC>
-__device__ __forceinline__ f4 ld4(const float* __restrict__ p, long long row, long long nrows,
-                                  long long cols, long long c) {
-    f4 r = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (row < nrows) {
-        const float* src = p + row * cols;
-        if (VEC) {
-            if (c < cols) r = *(const f4*)(src + c);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (c + e < cols) r[e] = src[c + e];
-        }
-    }
-    return r;
-}
-
-// m <= 16: one workgroup per 16 rows; wave w takes slices w, w+W, w+2W, ... four at a
-// time, loading them before their chains start (four independent chains interleave);
-// slice partials meet in LDS and one pass adds them in order.
-// Row `row`, columns c .. c + 3 of fp16 weights (cols a multiple of 64), widened; zeros past
-// the last row.
-__device__ __forceinline__ f4 ld4w16(const float* __restrict__ p, long long row, long long nrows,
-                                     long long cols, long long c) {
-    f4 r = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (row < nrows && c < cols) r = wide4(*(const h4*)((const _Float16*)p + row * cols + c));
-    return r;
-}
-
-template <bool VEC, bool H, bool W16 = false>
-__device__ void linear_small_body(float* __restrict__ y, const float* __restrict__ w,
-                                  const float* __restrict__ x, int rows, int cols, int m) {
-    extern __shared__ float part[];  // [slices][16 rows][16 tokens]
-    int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-    int i = lane & 15, g = lane >> 4;
-    long long r0 = (long long)blockIdx.x * 16;
-    int kblocks = (cols + 15) >> 4, nsl = (kblocks + SLM_KS - 1) / SLM_KS;
-    for (int s0 = wave; s0 < nsl; s0 += 4 * waves) {
-        f4 wa[4][SLM_KS], xb[4][SLM_KS];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            int s = s0 + j * waves;
-#pragma unroll
-            for (int u = 0; u < SLM_KS; u++) {
-                int kb = s * SLM_KS + u;
-                wa[j][u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-                xb[j][u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-                if (s < nsl && kb < kblocks) {
-                    long long c = (long long)kb * 16 + g * 4;
-                    if constexpr (W16) wa[j][u] = ld4w16(w, r0 + i, rows, cols, c);
-                    else wa[j][u] = ld4<VEC>(w, r0 + i, rows, cols, c);
-                    xb[j][u] = ld4<VEC>(x, i, m, cols, c);
-                }
-            }
-        }
-        f4 acc[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-        if constexpr (H) {
-#pragma unroll
-            for (int u = 0; u < SLM_KS; u++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    int s = s0 + j * waves;
-                    if (s < nsl && s * SLM_KS + u < kblocks) acc[j] = block16h(wa[j][u], xb[j][u], acc[j]);
-                }
-        } else {
-#pragma unroll
-            for (int u = 0; u < SLM_KS; u++)
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        int s = s0 + j * waves;
-                        if (s < nsl && s * SLM_KS + u < kblocks) acc[j] = mfma4(wa[j][u][e], xb[j][u][e], acc[j]);
-                    }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            int s = s0 + j * waves;
-            if (s < nsl) {
-#pragma unroll
-                for (int r = 0; r < 4; r++) part[s * 256 + (4 * g + r) * 16 + i] = acc[j][r];
-            }
-        }
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < 256; t += blockDim.x) {
-        int rr = t >> 4, tt = t & 15;
-        float tot = 0.0f;
-        for (int s0 = 0; s0 < nsl; s0 += SLM_SPLIT) {
-            float q = part[s0 * 256 + t];
-            int s1 = min(s0 + SLM_SPLIT, nsl);
-            for (int s = s0 + 1; s < s1; s++) q = q + part[s * 256 + t];
-            tot = s0 == 0 ? q : tot + q;
-        }
-        if (r0 + rr < rows && tt < m) y[(long long)tt * rows + r0 + rr] = h16<H>(tot);
-    }
-}
-
-KERNEL void __launch_bounds__(512) slm_linear_small_v(float* y, const float* w, const float* x,
-                                                      int rows, int cols, int m) {
-    linear_small_body<true, false>(y, w, x, rows, cols, m);
-}
-KERNEL void __launch_bounds__(512) slm_linear_small_s(float* y, const float* w, const float* x,
-                                                      int rows, int cols, int m) {
-    linear_small_body<false, false>(y, w, x, rows, cols, m);
-}
-KERNEL void __launch_bounds__(512) slm_linear_small_vh(float* y, const float* w, const float* x,
-                                                       int rows, int cols, int m) {
-    linear_small_body<true, true>(y, w, x, rows, cols, m);
-}
-// fp16 mode with the weights stored as halves (w: rows x cols fp16)
-KERNEL void __launch_bounds__(512) slm_linear_small_vhw(float* y, const float* w, const float* x,
-                                                        int rows, int cols, int m) {
-    linear_small_body<true, true, true>(y, w, x, rows, cols, m);
-}
-
-// m > 16: a 64-row × 64-token tile per workgroup, 32 × 32 per wave (2 × 2 MFMA tiles).
-template <bool VEC>
-__device__ void linear_big_body(float* __restrict__ y, const float* __restrict__ w,
-                                const float* __restrict__ x, int rows, int cols, int m) {
-    int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int i = lane & 15, g = lane >> 4;
-    long long rb = (long long)blockIdx.x * 64 + (wave & 1) * 32;
-    long long tb = (long long)blockIdx.y * 64 + (wave >> 1) * 32;
-    int kblocks = (cols + 15) >> 4, nsl = (kblocks + SLM_KS - 1) / SLM_KS;
-    f4 tot[2][2], sp[2][2];
-    for (int s = 0; s < nsl; s++) {
-        f4 acc[2][2];
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int v = 0; v < 2; v++) acc[u][v] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-        int kb1 = min(s * SLM_KS + SLM_KS, kblocks);
-        for (int kb = s * SLM_KS; kb < kb1; kb++) {
-            long long c = (long long)kb * 16 + g * 4;
-            f4 a[2], b[2];
-#pragma unroll
-            for (int u = 0; u < 2; u++) a[u] = ld4<VEC>(w, rb + 16 * u + i, rows, cols, c);
-#pragma unroll
-            for (int v = 0; v < 2; v++) b[v] = ld4<VEC>(x, tb + 16 * v + i, m, cols, c);
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-#pragma unroll
-                    for (int v = 0; v < 2; v++) acc[u][v] = mfma4(a[u][e], b[v][e], acc[u][v]);
-        }
-        bool open = s % SLM_SPLIT == 0, close = s % SLM_SPLIT == SLM_SPLIT - 1 || s == nsl - 1;
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int v = 0; v < 2; v++) {
-                sp[u][v] = open ? acc[u][v] : sp[u][v] + acc[u][v];
-                if (close) tot[u][v] = s < SLM_SPLIT ? sp[u][v] : tot[u][v] + sp[u][v];
-            }
-    }
-#pragma unroll
-    for (int u = 0; u < 2; u++)
-#pragma unroll
-        for (int v = 0; v < 2; v++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                long long row = rb + 16 * u + 4 * g + r, tok = tb + 16 * v + i;
-                if (row < rows && tok < m) y[tok * rows + row] = tot[u][v][r];
-            }
-}
-
-KERNEL void __launch_bounds__(256) slm_linear_big_v(float* y, const float* w, const float* x,
-                                                    int rows, int cols, int m) {
-    linear_big_body<true>(y, w, x, rows, cols, m);
-}
-KERNEL void __launch_bounds__(256) slm_linear_big_s(float* y, const float* w, const float* x,
-                                                    int rows, int cols, int m) {
-    linear_big_body<false>(y, w, x, rows, cols, m);
-}
-
-// m > 16, columns a multiple of 4, 16-byte aligned rows: the prompt GEMM. A 64-row × 64-token
-// tile per workgroup, 32 × 32 per wave; the weights and tokens of one slice (64 columns)
+// More tokens, columns not a multiple of 64 (slm_gemm: a multiple of 4, 16-byte aligned rows;
+// slm_gemm_s: any, loaded one float at a time). A 64-row × 64-token tile per workgroup, 32 × 32 per wave; the weights and tokens of one slice (64 columns)
 // at a time are staged in LDS (row stride 68 floats), the next slice's loads in flight
 // while one computes. blockIdx.z is the split: with several splits each workgroup adds
 // one split's slices and writes its partial to part[split][token][row] (added in order by
-// slm_fold); with one it writes y. Same chain and sums as linear_big_body.
+// slm_fold); with one it writes y, adding the splits itself. The canonical chain.
 #define GEMM_LS 68
-KERNEL void __launch_bounds__(256) slm_gemm(float* __restrict__ y, float* __restrict__ part,
-                                            const float* __restrict__ w,
-                                            const float* __restrict__ x, int rows, int cols,
-                                            int m) {
+template <bool VEC>
+__device__ __forceinline__ void gemm_body(float* __restrict__ y, float* __restrict__ part,
+                                          const float* __restrict__ w, const float* __restrict__ x,
+                                          int rows, int cols, int m) {
     __shared__ float sw[2][64 * GEMM_LS];
     __shared__ float sx[2][64 * GEMM_LS];
     int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1110,18 +932,27 @@ KERNEL void __launch_bounds__(256) slm_gemm(float* __restrict__ y, float* __rest
     int wr = (wave & 1) * 32, wt = (wave >> 1) * 32;
     long long r0 = (long long)blockIdx.x * 64, t0 = (long long)blockIdx.y * 64;
     int kblocks = (cols + 15) >> 4, nsl = (kblocks + SLM_KS - 1) / SLM_KS;
-    int s_first = blockIdx.z * SLM_SPLIT, s_end = min(nsl, s_first + SLM_SPLIT);
+    int s_first = blockIdx.z * SLM_SPLIT, s_end = gridDim.z > 1 ? min(nsl, s_first + SLM_SPLIT) : nsl;
     // staging: f4 number fi = tid + 256q of a 64 x 64 tile: row fi / 16, column 4 (fi % 16)
     f4 rw[4], rx[4];
     auto fetch = [&](int s) {
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             int fi = tid + 256 * q, row = fi >> 4, c = s * 64 + 4 * (fi & 15);
-            bool cin = c < cols;
+            bool cin = c < cols, wok = r0 + row < rows, xok = t0 + row < m;
             rw[q] = f4{0.0f, 0.0f, 0.0f, 0.0f};
             rx[q] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (cin && r0 + row < rows) rw[q] = *(const f4*)(w + (r0 + row) * cols + c);
-            if (cin && t0 + row < m) rx[q] = *(const f4*)(x + (t0 + row) * cols + c);
+            if constexpr (VEC) {
+                if (cin && wok) rw[q] = *(const f4*)(w + (r0 + row) * cols + c);
+                if (cin && xok) rx[q] = *(const f4*)(x + (t0 + row) * cols + c);
+            } else {
+                const float *pw = w + (wok ? (r0 + row) * cols : 0), *px = x + (xok ? (t0 + row) * cols : 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    rw[q][e] = gld(wok && c + e < cols ? pw + c + e : slm_zero16);
+                    rx[q][e] = gld(xok && c + e < cols ? px + c + e : slm_zero16);
+                }
+            }
         }
     };
     auto stash = [&](int b) {
@@ -1166,21 +997,21 @@ KERNEL void __launch_bounds__(256) slm_gemm(float* __restrict__ y, float* __rest
 #pragma unroll
                     for (int v = 0; v < 2; v++) acc[u][v] = mfma4(a[u][e], bb[v][e], acc[u][v]);
         }
-        // slice sums in order within the split, split sums in order (one split here)
-        bool open = (s - s_first) == 0;
+        // slice sums in order within the split, split sums in order
+        int in = (s - s_first) % SLM_SPLIT;
+        bool open = in == 0, close = in == SLM_SPLIT - 1 || s == s_end - 1, first = s - s_first < SLM_SPLIT;
 #pragma unroll
         for (int u = 0; u < 2; u++)
 #pragma unroll
-            for (int v = 0; v < 2; v++) sp[u][v] = open ? acc[u][v] : sp[u][v] + acc[u][v];
+            for (int v = 0; v < 2; v++) {
+                sp[u][v] = open ? acc[u][v] : sp[u][v] + acc[u][v];
+                if (close) tot[u][v] = first ? sp[u][v] : tot[u][v] + sp[u][v];
+            }
         if (s + 1 < s_end) {
             stash(b ^ 1);
             __syncthreads();
         }
     }
-#pragma unroll
-    for (int u = 0; u < 2; u++)
-#pragma unroll
-        for (int v = 0; v < 2; v++) tot[u][v] = sp[u][v];
     // out: D[4g + r][i] is row wr + 16u + 4g + r, token wt + 16v + i; through LDS so the
     // stores run along rows
     __syncthreads();
@@ -1197,6 +1028,14 @@ KERNEL void __launch_bounds__(256) slm_gemm(float* __restrict__ y, float* __rest
         int tok = e >> 6, row = e & 63;
         if (t0 + tok < m && r0 + row < rows) out[(t0 + tok) * rows + r0 + row] = so[tok * 65 + row];
     }
+}
+KERNEL void __launch_bounds__(256) slm_gemm(float* y, float* part, const float* w, const float* x,
+                                            int rows, int cols, int m) {
+    gemm_body<true>(y, part, w, x, rows, cols, m);
+}
+KERNEL void __launch_bounds__(256) slm_gemm_s(float* y, float* part, const float* w, const float* x,
+                                              int rows, int cols, int m) {
+    gemm_body<false>(y, part, w, x, rows, cols, m);
 }
 
 // The same GEMM with a deeper pipeline, for cols a multiple of 64 and 16-byte aligned rows:
@@ -1593,6 +1432,239 @@ __device__ void gemm2_body(float* __restrict__ y, float* __restrict__ part,
         if (t0 + tok < m && r0 + row < rows) out[(t0 + tok) * rows + r0 + row] = so[tok * (BM + 1) + row];
     }
 }
+
+// Few tokens (up to 32): a workgroup takes one row tile of 16·RW rows for 16·NV tokens and every
+// slice of its columns at once, a slice a wave at a time: the wave's weights and tokens come
+// straight into registers (nothing is staged, no barrier until the slices are done), the slice
+// partials meet in LDS and one pass adds them in order. What bounds these shapes is latency, not
+// rate: the prompt GEMMs below walk a split's twelve slices one after another through LDS, a
+// memory round trip each (a 21-token 2304 x 768 projection 20 us); here all twelve are in
+// flight together. Each workgroup reads all its tokens, so past 32 tokens the GEMMs, whose tiles
+// share them, are the faster. 768 x 3072 at 5 tokens 13.8 -> 7.4 us (with the launch that adds its
+// four splits), 2304 x 768 5.3 -> 4.3; 2304 x 768 with the attention epilogue at 21 tokens 20 -> 7.
+// EPI 0: y [m][rows] (or, with several splits in blockIdx.z, part[split][m][rows]); rt rows a
+// tile (16, 8 or 4: a short matrix spreads over more CUs; the other MFMA rows are zeros).
+// EPI 1: the SiLU pair (tile rows i and i + 8 are gate and amp), as gemm2's SILU. EPI 2: the
+// attention input (tile rows i and i + 8 are a head's rope pair), as gemm2's ROPE 1. EPI 3 (RW =
+// 4): the linear-attention input, a head of 64 rows a tile, as gemm2's ROPE 2. The arithmetic is
+// the canonical chain.
+// VEC false (EPI 0, fp32): single floats, any number of columns and any alignment.
+template <int NV, bool H, bool W16, int EPI, bool VEC = true>
+__device__ __forceinline__ void linear_small_body(float* __restrict__ y, float* __restrict__ part,
+                             const float* __restrict__ w, const float* __restrict__ x, int rows,
+                             int cols, int m, int rt, GemmEpi ep = GemmEpi{}) {
+    static_assert(!W16 || H, "fp16 weights run the fp16 chain");
+    constexpr int RW = EPI == 3 ? 4 : 1, TR = 16 * RW, NTOK = 16 * NV;
+    constexpr int J = NV == 1 ? 3 : NV == 2 ? 2 : 1;  // slices in flight a wave (128 registers)
+    extern __shared__ __attribute__((aligned(16))) float lds[];  // [slices][NTOK][TR], then [NTOK][TR + 1]
+    int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int waves = blockDim.x >> 6, i = lane & 15, g = lane >> 4;
+    int wt = RW == 1 ? 0 : wave % RW, w0 = RW == 1 ? wave : wave / RW, ws = waves / RW;
+    long long t0 = (long long)blockIdx.y * NTOK;
+    int kblocks = (cols + 15) >> 4, nsl = (kblocks + SLM_KS - 1) / SLM_KS;
+    int s_first = gridDim.z > 1 ? blockIdx.z * SLM_SPLIT : 0, s_end = gridDim.z > 1 ? min(nsl, s_first + SLM_SPLIT) : nsl;
+    long long half = rows / 2;
+    // the matrix row of tile row r (rows: none)
+    auto row_of = [&](int r) -> long long {
+        if (EPI == 1) {
+            long long j = (long long)blockIdx.x * 8 + (r & 7);
+            return j < half ? (r < 8 ? j : half + j) : rows;
+        }
+        if (EPI == 2) return (long long)(blockIdx.x >> 2) * 64 + 8 * (blockIdx.x & 3) + (r < 8 ? r : 24 + r);
+        if (EPI == 3) return (long long)blockIdx.x * 64 + r;
+        long long v = (long long)blockIdx.x * rt + r;
+        return r < rt && v < rows ? v : rows;
+    };
+    long long wr = row_of(16 * wt + i);
+    bool rok = wr < rows;
+    const float* wrow = w + (rok ? wr * cols : 0);
+    const _Float16* hrow = (const _Float16*)w + (rok ? wr * cols : 0);
+    const float* xrow[NV];
+    bool tok_ok[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+        long long t = t0 + 16 * v + i;
+        tok_ok[v] = t < m;
+        xrow[v] = x + (tok_ok[v] ? t * cols : 0);
+    }
+    for (int sa = s_first + w0; sa < s_end; sa += J * ws) {
+        f4 a[J][SLM_KS], b[J][SLM_KS][NV];
+        h4 aw[J][SLM_KS];
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            int s = sa + j * ws;
+            if (s >= s_end) break;
+#pragma unroll
+            for (int u = 0; u < SLM_KS; u++) {
+                int c = s * 64 + 16 * u + 4 * g;
+                bool in = c < cols;
+                if constexpr (!VEC) {  // single floats: any number of columns, any alignment
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        bool ine = c + e < cols;
+                        a[j][u][e] = gld(ine && rok ? wrow + c + e : slm_zero16);
+#pragma unroll
+                        for (int v = 0; v < NV; v++) b[j][u][v][e] = gld(ine && tok_ok[v] ? xrow[v] + c + e : slm_zero16);
+                    }
+                    continue;
+                }
+                if constexpr (W16) aw[j][u] = gld((const h4*)(in && rok ? hrow + c : (const _Float16*)slm_zero16));
+                else a[j][u] = gld((const f4*)(in && rok ? wrow + c : slm_zero16));
+#pragma unroll
+                for (int v = 0; v < NV; v++) b[j][u][v] = gld((const f4*)(in && tok_ok[v] ? xrow[v] + c : slm_zero16));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every load is out before the first MFMA
+        f4 acc[J][NV];
+#pragma unroll
+        for (int j = 0; j < J; j++)
+#pragma unroll
+            for (int v = 0; v < NV; v++) acc[j][v] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        auto chain = [&](int j) {
+#pragma unroll
+            for (int u = 0; u < SLM_KS; u++) {
+                if constexpr (H) {
+#pragma unroll
+                    for (int v = 0; v < NV; v++) {
+                        if constexpr (W16) acc[j][v] = block16hw(aw[j][u], b[j][u][v], acc[j][v]);
+                        else acc[j][v] = block16h(a[j][u], b[j][u][v], acc[j][v]);
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+#pragma unroll
+                        for (int v = 0; v < NV; v++) acc[j][v] = mfma4(a[j][u][e], b[j][u][v][e], acc[j][v]);
+                }
+            }
+        };
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            int s = sa + j * ws;
+            if (s >= s_end) break;
+            chain(j);
+#pragma unroll
+            for (int v = 0; v < NV; v++)
+                *(f4*)(lds + ((s - s_first) * NTOK + 16 * v + i) * TR + 16 * wt + 4 * g) = acc[j][v];
+        }
+    }
+    __syncthreads();
+    // the slice sums of a split in order, the splits in order
+    float* so = lds + (s_end - s_first) * NTOK * TR;  // [NTOK][TR + 1]
+    auto total = [&](int e) {
+        float tot = 0.0f;
+        for (int s0 = s_first; s0 < s_end; s0 += SLM_SPLIT) {
+            const float* p = lds + (s0 - s_first) * NTOK * TR + e;
+            int n = min(SLM_SPLIT, s_end - s0);
+            float pv[SLM_SPLIT];
+#pragma unroll
+            for (int k = 0; k < SLM_SPLIT; k++) pv[k] = p[min(k, n - 1) * NTOK * TR];
+            float q = pv[0];
+#pragma unroll
+            for (int k = 1; k < SLM_SPLIT; k++) q = k < n ? q + pv[k] : q;
+            tot = s0 == s_first ? q : tot + q;
+        }
+        // (fp16 mode: the linear's output rounded; a split's partials are not)
+        return H && gridDim.z == 1 ? r16(tot) : tot;
+    };
+    if constexpr (EPI == 0) {
+        float* out = gridDim.z > 1 ? part + (long long)blockIdx.z * m * rows : y;
+        for (int e = tid; e < NTOK * 16; e += blockDim.x) {
+            long long row = row_of(e & 15), t = t0 + (e >> 4);
+            if (row < rows && t < m) out[t * rows + row] = total(e);
+        }
+        return;
+    }
+    for (int e = tid; e < NTOK * TR; e += blockDim.x)
+        if (t0 + e / TR < m) so[(e / TR) * (TR + 1) + e % TR] = total(e);
+    __syncthreads();
+    if constexpr (EPI == 1) {
+        for (int e = tid; e < NTOK * 8; e += blockDim.x) {
+            long long j = (long long)blockIdx.x * 8 + (e & 7), t = t0 + (e >> 3);
+            const float* sr = so + (e >> 3) * 17;
+            if (t < m && j < half) y[t * half + j] = e_silu<H>(sr[e & 7], sr[8 + (e & 7)]);
+        }
+    }
+    if constexpr (EPI == 2) {
+        // (heads of 64: a quarter of a head's rope pairs a tile, slm_gemm2r_64's expressions)
+        long long r0 = (long long)(blockIdx.x >> 2) * 64;
+        int sub = 8 * (blockIdx.x & 3), region = (int)(r0 / ep.d), head = (int)((r0 % ep.d) >> 6);
+        long long pos = 0;
+        if (region == 1) pos = ep.kdyn ? ep.kdyn[0] : ep.kpos;
+        if (region == 2) pos = ep.vdyn ? ep.vdyn[0] : ep.vpos;
+        float* dst = region == 0 ? ep.q : region == 1 ? ep.k : ep.v;
+        float* ring = region == 1 ? ep.kring : ep.vring;
+        for (int e = tid; e < NTOK * 16; e += blockDim.x) {
+            int r = e & 15, ie = sub + (r & 7), j = r < 8 ? ie : 32 + ie;
+            long long t = t0 + (e >> 4);
+            if (t >= m) continue;
+            const float* sr = so + (e >> 4) * 17;
+            float v = sr[r];
+            y[t * rows + r0 + j] = v;
+            if (region < 2) {
+                float c = ep.cs[t * 32 + ie], sn = ep.sn[t * 32 + ie], a = sr[r & 7], b = sr[8 + (r & 7)];
+                v = r < 8 ? e_rope_l<H>(a, b, c, sn) : e_rope_r<H>(a, b, c, sn);
+            }
+            dst[t * ep.d + head * 64 + j] = v;
+            if (region > 0) {
+                long long at = ((long long)head * ep.cap + (pos + t) % ep.cap) * 64 + j;
+                if (ep.ring16) ((_Float16*)ring)[at] = (_Float16)v;
+                else ring[at] = v;
+            }
+        }
+    }
+    if constexpr (EPI == 3) {
+        long long r0 = (long long)blockIdx.x * 64;
+        int region = (int)(r0 / ep.d), head = (int)((r0 % ep.d) >> 6);
+        float* dst = region == 0 ? ep.q : region == 1 ? ep.k : region == 2 ? ep.v : ep.g;
+        for (int tok = wave; tok < NTOK; tok += waves) {
+            long long t = t0 + tok;
+            if (t >= m) break;
+            const float* sr = so + tok * 65;
+            float v = sr[lane];
+            y[t * rows + r0 + lane] = v;
+            if (region < 2) v = h16<H>(v * (1.0f / fmaxf(sqrtf(dot16_wave(sr, 64, lane)), 1e-12f)));
+            dst[t * ep.d + head * 64 + lane] = v;
+        }
+    }
+}
+
+#define LSMALL_K(NAME, NV, H, W16, VEC)                                                                       \
+    KERNEL void __launch_bounds__(1024) NAME(float* y, float* part, const float* w, const float* x,   \
+                                             int rows, int cols, int m, int rt) {                      \
+        linear_small_body<NV, H, W16, 0, VEC>(y, part, w, x, rows, cols, m, rt);                                \
+    }
+#define LSMALLS_K(NAME, NV, H, W16)                                                                      \
+    KERNEL void __launch_bounds__(1024) NAME(float* y, float* part, const float* w, const float* x,   \
+                                             int rows, int cols, int m) {                              \
+        linear_small_body<NV, H, W16, 1>(y, part, w, x, rows, cols, m, 16);                                \
+    }
+#define LSMALLR_K(NAME, NV, H, W16)                                                                      \
+    KERNEL void __launch_bounds__(1024)                                                               \
+        NAME(float* y, float* part, const float* w, const float* x, int rows, int cols, int m,         \
+             float* q, float* k, float* v, float* kring, float* vring, const float* cs,                \
+             const float* sn, const long long* kdyn, const long long* vdyn, long long kpos,           \
+             long long vpos, long long cap, int d, int ring16) {                                       \
+        linear_small_body<NV, H, W16, 2>(y, part, w, x, rows, cols, m, 16,                                 \
+            GemmEpi{q, k, v, kring, vring, cs, sn, nullptr, kdyn, vdyn, kpos, vpos, cap, d, ring16});  \
+    }
+#define LSMALLN_K(NAME, NV, H, W16)                                                                      \
+    KERNEL void __launch_bounds__(1024)                                                               \
+        NAME(float* y, float* part, const float* w, const float* x, int rows, int cols, int m,         \
+             float* q, float* k, float* v, float* g, int d) {                                          \
+        linear_small_body<NV, H, W16, 3>(y, part, w, x, rows, cols, m, 16,                                 \
+            GemmEpi{q, k, v, nullptr, nullptr, nullptr, nullptr, g, nullptr, nullptr, 0, 0, 0, d, 0}); \
+    }
+#define LSMALL(NV)                                                                                       \
+    LSMALL_K(slm_linear_small_v_##NV, NV, false, false, true) LSMALL_K(slm_linear_small_s_##NV, NV, false, false, false)            \
+    LSMALL_K(slm_linear_small_vh_##NV, NV, true, false, true) LSMALL_K(slm_linear_small_vhw_##NV, NV, true, true, true)          \
+    LSMALLS_K(slm_linear_smalls_##NV, NV, false, false) LSMALLS_K(slm_linear_smallsh_##NV, NV, true, false) LSMALLS_K(slm_linear_smallshw_##NV, NV, true, true) \
+    LSMALLR_K(slm_linear_smallr_##NV, NV, false, false) LSMALLR_K(slm_linear_smallrh_##NV, NV, true, false) LSMALLR_K(slm_linear_smallrhw_##NV, NV, true, true)
+LSMALL(1)
+LSMALL(2)
+#define LSMALLN(NV)                                                                                      \
+    LSMALLN_K(slm_linear_smalln_##NV, NV, false, false) LSMALLN_K(slm_linear_smallnh_##NV, NV, true, false) LSMALLN_K(slm_linear_smallnhw_##NV, NV, true, true)
+LSMALLN(1)
+LSMALLN(2)
 
 #define GEMM2_K(NAME, BM, WAVES, H, S, W16)                                               \
     KERNEL void __launch_bounds__(64 * WAVES) NAME(float* y, float* part, const float* w,  \

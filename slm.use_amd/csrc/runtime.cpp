@@ -127,10 +127,9 @@ struct Kernels {
     hipFunction_t copy, add, add_row, mix, silu_mul, scale_rows, shift, columns, gather,
         store, rope, rope_table, rms, l2norm, rms_wave, l2norm_wave, fill, combine, probe, fg, fold,
         gemm, gemm2_32, gemm2_64, gemm2_96, gemm2_128, gemm2h_32, gemm2h_64, gemm2h_96, gemm2h_128,
-        lin_small_h, fgh;
+        gemm_s, fgh;
     // fp16 mode over fp16 weights (allocated with slm_hip_alloc_half)
-    hipFunction_t lin_small_hw, fghw, gemm2hw[4], gemm2hsw[4], gemm2hrw, gemm2hnw;
-    hipFunction_t lin_small[2], lin_big[2];  // [vec]
+    hipFunction_t fghw, gemm2hw[4], gemm2hsw[4], gemm2hrw, gemm2hnw;
     hipFunction_t gla[5], gla1[3];           // head sizes to 16, 32, .. 256; one token: to 16, 32, 64
     hipFunction_t glah[5];                   // the prompt GLA in fp16 mode
     hipFunction_t attn[5];                   // dim tiles 1, 2, 4, 8, 16
@@ -139,6 +138,9 @@ struct Kernels {
     hipFunction_t gemm2s[4], gemm2hs[4];     // prompt GEMM with the SiLU pair epilogue, BM 32..128
     hipFunction_t gemm2r, gemm2hr;           // prompt QKV GEMM with the rope + ring-store epilogue
     hipFunction_t gemm2n, gemm2hn;           // prompt QKVG GEMM with the per-head L2 epilogue
+    // few tokens, by 16-token blocks: [0] fp32, [1] fp16 mode, [2] fp16 weights; plain, SiLU pair,
+    // attention input, linear-attention input; plain fp32 for any columns and alignment
+    hipFunction_t lin_small[3][2], lin_smalls[3][2], lin_smallr[3][2], lin_smalln[3][2], lin_small1[2];
     hipFunction_t rows;                      // prompt row chains
     hipFunction_t attn_pq[3];                // prompt attention, superblock shared in LDS
     hipFunction_t gemm2k_32, gemm2k_16;      // 32- and 16-row tiles, two slice groups (fp32)
@@ -636,6 +638,17 @@ int gemm2_bm_plain(int64_t rows, int64_t m, int64_t ns) {
     return bm;
 }
 
+// The few-token kernels (slm_linear_small*), up to SMALL_M tokens. Every workgroup reads all the
+// tokens, so their time grows with them: 2304 x 768 took 4.3 us at 5 tokens, 6.6 at 32, 8.7 at 48,
+// 10.7 at 64, the GEMMs, which walk the columns through LDS, 7.7 to 7.9 from 17 to 64 (6144 x 768:
+// 7.0, 11.9, 15.7, 19.0 against 11.2 to 11.5).
+constexpr int64_t SMALL_M = 32;
+int small_nv(int64_t m) { return (int)((std::min<int64_t>(m, SMALL_M) + 15) / 16); }  // 16-token blocks
+int small_type(const Op& L) { return L.n[4] ? 2 : L.n[3] ? 1 : 0; }
+// LDS floats of `slices` slice partials and the epilogue's tile, `tr` tile rows
+int64_t small_lds(int64_t slices, int nv, int tr) { return slices * 16 * nv * tr + 16 * nv * (tr + 1); }
+uint32_t small_waves(int64_t slices) { return (uint32_t)std::min<int64_t>(slices, 16); }
+
 // A linear (p0 y, p1 w, p2 x; n0 rows, n1 cols, n2 m). With `fold_ns`, a split GEMM's
 // partials are left in c->gpart for the caller to add (*fold_ns: the split count, 1 when
 // the GEMM wrote y itself).
@@ -656,27 +669,49 @@ int lower_linear(slm_hip* c, const Op& o, std::vector<Rec>& out, int64_t* fold_n
     bool h = n[3] != 0;  // fp16 mode: 64-column multiples, aligned (checked when recorded)
     bool w16 = n[4] != 0;  // fp16 weights (fp16 mode)
     if (w16) ab = 2.0 * (double)(rows * cols) + 4.0 * (double)(m * cols + m * rows);
-    if (h && m <= 16 && nsl <= 64) {
-        uint32_t waves = (uint32_t)std::min<int64_t>(nsl, 8);
-        out.push_back(mk(w16 ? k.lin_small_hw : k.lin_small_h, (uint32_t)((rows + 15) / 16), 1, 1, 64 * waves,
-                         (uint32_t)(nsl * 1024), p[0], p[1], p[2], (int)rows, (int)cols, (int)m));
-        out.back().abytes = ab;
-        return SLM_OK;
-    }
-    if (h && (m <= 16 || !vec || cols % 64))
+    if (h && (!vec || cols % 64 || (m <= 16 && nsl > 64)))
         return fail(c, SLM_E_UNSUPPORTED, "linear: fp16 mode has no kernel for %lld x %lld x %lld",
                     (long long)rows, (long long)cols, (long long)m);
-    if (m <= 16 && nsl <= 64) {
-        uint32_t waves = (uint32_t)std::min<int64_t>(nsl, 8);
-        out.push_back(mk(k.lin_small[vec], (uint32_t)((rows + 15) / 16), 1, 1, 64 * waves,
-                         (uint32_t)(nsl * 1024), p[0], p[1], p[2], (int)rows, (int)cols,
-                         (int)m));
-        out.back().abytes = ab;
-    } else if (vec) {  // the LDS-staged GEMM, one workgroup column per split
+    if (m <= SMALL_M) {
+        int nv = small_nv(m);
         int64_t ns = (nsl + SLM_SPLIT - 1) / SLM_SPLIT;
-        if (ns > 1 && (int64_t)c->gpart_bytes < ns * m * rows * 4)
-            return fail(c, SLM_E_INVALID, "linear: no room for %lld split partials", (long long)ns);
-        if (cols % 64 == 0) {
+        // one launch over all the splits where their partials fit in LDS, or a split in each
+        // blockIdx.z (always where the caller adds the partials). The busiest CU's time, us: its
+        // weights and tokens at 50 KB/us, its MFMAs (sixteen rows whatever the tile holds), and
+        // 1.7 for the launch that adds the partials (measured, 768 x 3072: one launch 9.4 us at 5
+        // tokens, 11.6 at 16, 18.6 at 32; a split a workgroup and the sum 7.7 at 16, 9.3 at 32)
+        double best = -1.0;
+        int rt = 16;
+        int64_t z = 1;
+        auto consider = [&](int64_t zs, double extra) {
+            int64_t per = zs > 1 ? SLM_SPLIT : nsl;
+            for (int t : {16, 8, 4}) {
+                double wgs = std::ceil((double)((rows + t - 1) / t * zs) / CU_COUNT);
+                double us = extra + wgs * (256.0 * (double)per * (double)(t + m) / 50e3 + (double)(per * nv) * 16 * 36 / 4 / 2.4e3);
+                if (best < 0 || us < (t == 16 ? best : 0.9 * best)) best = us, rt = t, z = zs;
+            }
+        };
+        bool room = (int64_t)c->gpart_bytes >= ns * m * rows * 4;
+        if (ns == 1 || (!fold_ns && 4 * small_lds(nsl, nv, 16) <= LDS_MAX)) consider(1, 0.0);
+        if (ns > 1 && room) consider(ns, fold_ns ? 0.0 : 1.7);
+        if (best < 0) return fail(c, SLM_E_INVALID, "linear: no room for %lld split partials", (long long)ns);
+        int64_t per = z > 1 ? SLM_SPLIT : nsl;
+        out.push_back(mk(vec ? k.lin_small[small_type(o)][nv - 1] : k.lin_small1[nv - 1], (uint32_t)((rows + rt - 1) / rt), 1, (uint32_t)z,
+                         64 * small_waves(per), (uint32_t)(4 * small_lds(per, nv, 16)), p[0], c->gpart, p[1], p[2],
+                         (int)rows, (int)cols, (int)m, rt));
+        out.back().abytes = ab;
+        if (fold_ns) *fold_ns = z;
+        else if (z > 1)
+            out.push_back(mk(k.fold, blocks_for(m * rows), 1, 1, 256, 0, p[0],
+                             (const float*)c->gpart, (long long)(m * rows), (int)z));
+        return SLM_OK;
+    }
+    {  // the LDS-staged GEMMs, one workgroup column per split
+        int64_t ns = (nsl + SLM_SPLIT - 1) / SLM_SPLIT;
+        bool room = ns == 1 || (int64_t)c->gpart_bytes >= ns * m * rows * 4;
+        if (!room && vec) return fail(c, SLM_E_INVALID, "linear: no room for %lld split partials", (long long)ns);
+        if (!room) ns = 1;  // (slm_gemm_s then adds its splits itself)
+        if (vec && cols % 64 == 0) {
             // the tile rows by the chip's fill (in fp16 mode 32-row tiles run as 48: the slice
             // groups of 32 rows are fp32 only)
             int bm = gemm2_bm_plain(rows, m, ns);
@@ -697,7 +732,7 @@ int lower_linear(slm_hip* c, const Op& o, std::vector<Rec>& out, int64_t* fold_n
                              (uint32_t)ns, threads, shmem, p[0], c->gpart,
                              p[1], p[2], (int)rows, (int)cols, (int)m));
         } else {
-            out.push_back(mk(k.gemm, (uint32_t)((rows + 63) / 64), (uint32_t)((m + 63) / 64),
+            out.push_back(mk(vec ? k.gemm : k.gemm_s, (uint32_t)((rows + 63) / 64), (uint32_t)((m + 63) / 64),
                              (uint32_t)ns, 256, 0, p[0], c->gpart, p[1], p[2], (int)rows,
                              (int)cols, (int)m));
         }
@@ -705,10 +740,6 @@ int lower_linear(slm_hip* c, const Op& o, std::vector<Rec>& out, int64_t* fold_n
         else if (ns > 1)
             out.push_back(mk(k.fold, blocks_for(m * rows), 1, 1, 256, 0, p[0],
                              (const float*)c->gpart, (long long)(m * rows), (int)ns));
-    } else {
-        out.push_back(mk(k.lin_big[vec], (uint32_t)((rows + 63) / 64),
-                         (uint32_t)((m + 63) / 64), 1, 256, 0, p[0], p[1], p[2],
-                         (int)rows, (int)cols, (int)m));
     }
     return SLM_OK;
 }
@@ -2209,7 +2240,7 @@ struct Planner {
         if (i + 3 >= ops.size()) return 0;
         const Op &cg = ops[i + 1], &ca = ops[i + 2], &sm = ops[i + 3];
         int64_t rows = L.n[0], cols = L.n[1], m = L.n[2], h = rows / 2;
-        if (m <= 16 || rows % 2 || cols % 64 || cols / 64 > SLM_SPLIT || !aligned16(L.p[1]) ||
+        if (rows % 2 || cols % 64 || cols / 64 > SLM_SPLIT || !aligned16(L.p[1]) ||
             !aligned16(L.p[2]))
             return 0;
         if (cg.kind != OP_COLUMNS || ca.kind != OP_COLUMNS || sm.kind != OP_SILU_MUL) return 0;
@@ -2222,6 +2253,15 @@ struct Planner {
             return 0;
         Range ry = rng(sm.p[0], m * h);
         if (overlap(ry, rng(L.p[1], wfloats(L))) || overlap(ry, rng(L.p[2], m * cols))) return 0;
+        if (m <= SMALL_M) {
+            int nv = small_nv(m);
+            out.push_back(mk(c->k.lin_smalls[small_type(L)][nv - 1], (uint32_t)((h + 7) / 8), 1, 1, 64 * small_waves(cols / 64),
+                             (uint32_t)(4 * small_lds(cols / 64, nv, 16)), sm.p[0], c->gpart, L.p[1], L.p[2],
+                             (int)rows, (int)cols, (int)m));
+            out.back().abytes = 4.0 * (double)(rows * cols + m * cols + m * h);
+            last_m = m;
+            return 4;
+        }
         int bm = gemm2_bm(rows, m, 1);
         int q = bm == 32 ? 0 : bm == 64 ? 1 : bm == 96 ? 2 : 3;
         uint32_t shmem = (uint32_t)(GEMM_STAGES_HOST * (bm * (L.n[4] ? 32 : 64) + 64 * 64) * 4);
@@ -2247,7 +2287,7 @@ struct Planner {
             c3.kind != OP_COLUMNS || s1.kind != OP_STORE || s2.kind != OP_STORE)
             return 0;
         int64_t rows = L.n[0], cols = L.n[1], m = L.n[2], d = rows / 3;
-        if (m <= 16 || rows % 3 || d % 64 || cols % 64 || cols / 64 > SLM_SPLIT || !aligned16(L.p[1]) ||
+        if (rows % 3 || d % 64 || cols % 64 || cols / 64 > SLM_SPLIT || !aligned16(L.p[1]) ||
             !aligned16(L.p[2]))
             return 0;
         const float* mix = L.p[0];
@@ -2283,10 +2323,13 @@ struct Planner {
                 if (overlap(wr[a], x)) return 0;
         }
         if (!dead_after(ops, i + 8, rng(cy, m * d))) return 0;
-        uint32_t shmem = (uint32_t)(GEMM_STAGES_HOST * (64 * (L.n[4] ? 32 : 64) + 64 * 64) * 4);
-        hipFunction_t gf = L.n[4] ? c->k.gemm2hrw : L.n[3] ? c->k.gemm2hr : c->k.gemm2r;
-        out.push_back(mk(gf, (uint32_t)(rows / 64), (uint32_t)((m + 63) / 64),
-                         1, gemm2_threads(64), shmem, (float*)mix, c->gpart, L.p[1], L.p[2], (int)rows,
+        bool few = m <= SMALL_M;
+        int nv = small_nv(m);
+        uint32_t shmem = few ? (uint32_t)(4 * small_lds(cols / 64, nv, 16))
+                             : (uint32_t)(GEMM_STAGES_HOST * (64 * (L.n[4] ? 32 : 64) + 64 * 64) * 4);
+        hipFunction_t gf = few ? c->k.lin_smallr[small_type(L)][nv - 1] : L.n[4] ? c->k.gemm2hrw : L.n[3] ? c->k.gemm2hr : c->k.gemm2r;
+        out.push_back(mk(gf, (uint32_t)(rows / (few ? 16 : 64)), few ? 1 : (uint32_t)((m + 63) / 64),
+                         1, few ? 64 * small_waves(cols / 64) : gemm2_threads(64), shmem, (float*)mix, c->gpart, L.p[1], L.p[2], (int)rows,
                          (int)cols, (int)m, (float*)q, (float*)k, (float*)v, (float*)s1.p[0],
                          (float*)s2.p[0], r1.p[2], r1.p[3], (const long long*)s1.dyn, (const long long*)s2.dyn,
                          (long long)s1.n[4], (long long)s2.n[4], (long long)cap, (int)d, (int)s1.n[5]));
@@ -2307,7 +2350,7 @@ struct Planner {
             n2.kind != OP_L2NORM || c3.kind != OP_COLUMNS || c4.kind != OP_COLUMNS)
             return 0;
         int64_t rows = L.n[0], cols = L.n[1], m = L.n[2], d = rows / 4;
-        if (m <= 16 || rows % 4 || d % 64 || cols % 64 || cols / 64 > SLM_SPLIT || !aligned16(L.p[1]) ||
+        if (rows % 4 || d % 64 || cols % 64 || cols / 64 > SLM_SPLIT || !aligned16(L.p[1]) ||
             !aligned16(L.p[2]))
             return 0;
         const float* mix = L.p[0];
@@ -2332,10 +2375,13 @@ struct Planner {
                 if (overlap(wr[a], x)) return 0;
         }
         if (!dead_after(ops, i + 7, rng(cy, m * d))) return 0;
-        uint32_t shmem = (uint32_t)(GEMM_STAGES_HOST * (64 * (L.n[4] ? 32 : 64) + 64 * 64) * 4);
-        hipFunction_t gf = L.n[4] ? c->k.gemm2hnw : L.n[3] ? c->k.gemm2hn : c->k.gemm2n;
-        out.push_back(mk(gf, (uint32_t)(rows / 64), (uint32_t)((m + 63) / 64),
-                         1, gemm2_threads(64), shmem, (float*)mix, c->gpart, L.p[1], L.p[2], (int)rows,
+        bool few = m <= SMALL_M;
+        int nv = small_nv(m);
+        uint32_t shmem = few ? (uint32_t)(4 * small_lds(cols / 64, nv, 64))
+                             : (uint32_t)(GEMM_STAGES_HOST * (64 * (L.n[4] ? 32 : 64) + 64 * 64) * 4);
+        hipFunction_t gf = few ? c->k.lin_smalln[small_type(L)][nv - 1] : L.n[4] ? c->k.gemm2hnw : L.n[3] ? c->k.gemm2hn : c->k.gemm2n;
+        out.push_back(mk(gf, (uint32_t)(rows / 64), few ? 1 : (uint32_t)((m + 63) / 64),
+                         1, few ? 1024 : gemm2_threads(64), shmem, (float*)mix, c->gpart, L.p[1], L.p[2], (int)rows,
                          (int)cols, (int)m, (float*)q, (float*)k, (float*)v, (float*)g, (int)d));
         out.back().abytes = 4.0 * (double)(rows * cols + m * cols + m * rows + 4 * m * d);
         last_m = m;
@@ -3426,9 +3472,7 @@ int load_kernels(slm_hip* c) {
                {&k.gemm2_96, "slm_gemm2_96"},   {&k.gemm2_128, "slm_gemm2_128"},
                {&k.gemm2h_32, "slm_gemm2h_32"}, {&k.gemm2h_64, "slm_gemm2h_64"},
                {&k.gemm2h_96, "slm_gemm2h_96"}, {&k.gemm2h_128, "slm_gemm2h_128"},
-               {&k.lin_small_h, "slm_linear_small_vh"}, {&k.fgh, "slm_fgh"},
-               {&k.lin_small[0], "slm_linear_small_s"}, {&k.lin_small[1], "slm_linear_small_v"},
-               {&k.lin_big[0], "slm_linear_big_s"},     {&k.lin_big[1], "slm_linear_big_v"},
+               {&k.gemm_s, "slm_gemm_s"}, {&k.fgh, "slm_fgh"},
                {&k.gla[0], "slm_gla_16"},   {&k.gla[1], "slm_gla_32"},   {&k.gla[2], "slm_gla_64"},
                {&k.gla[3], "slm_gla_128"},   {&k.gla[4], "slm_gla_256"},
                {&k.glah[0], "slm_glah_16"}, {&k.glah[1], "slm_glah_32"}, {&k.glah[2], "slm_glah_64"},
@@ -3447,7 +3491,7 @@ int load_kernels(slm_hip* c) {
                {&k.gemm2hs[2], "slm_gemm2hs_96"}, {&k.gemm2hs[3], "slm_gemm2hs_128"},
                {&k.gemm2r, "slm_gemm2r_64"},      {&k.gemm2hr, "slm_gemm2hr_64"},
                {&k.gemm2n, "slm_gemm2n_64"},      {&k.gemm2hn, "slm_gemm2hn_64"},
-               {&k.lin_small_hw, "slm_linear_small_vhw"}, {&k.fghw, "slm_fghw"},
+               {&k.fghw, "slm_fghw"},
                {&k.gemm2hw[0], "slm_gemm2hw_32"}, {&k.gemm2hw[1], "slm_gemm2hw_64"},
                {&k.gemm2hw[2], "slm_gemm2hw_96"}, {&k.gemm2hw[3], "slm_gemm2hw_128"},
                {&k.gemm2hsw[0], "slm_gemm2hsw_32"}, {&k.gemm2hsw[1], "slm_gemm2hsw_64"},
@@ -3458,6 +3502,22 @@ int load_kernels(slm_hip* c) {
     for (auto& f : fns) {
         TRY(get_fn(c, f.f, f.n));
         c->fname[*f.f] = f.n;
+    }
+    auto get = [&](hipFunction_t* f, std::string name) {
+        TRY(get_fn(c, f, name.c_str()));
+        c->fname[*f] = name;
+        return (int)SLM_OK;
+    };
+    for (int nv = 0; nv < 2; nv++) {
+        std::string n = "_" + std::to_string(nv + 1);
+        for (int t = 0; t < 3; t++) {
+            std::string h = (t == 2 ? "hw" : t ? "h" : "") + n;
+            TRY(get(&k.lin_small[t][nv], "slm_linear_small_v" + h));
+            TRY(get(&k.lin_smalls[t][nv], "slm_linear_smalls" + h));
+            TRY(get(&k.lin_smallr[t][nv], "slm_linear_smallr" + h));
+            TRY(get(&k.lin_smalln[t][nv], "slm_linear_smalln" + h));
+        }
+        TRY(get(&k.lin_small1[nv], "slm_linear_small_s" + n));
     }
     return SLM_OK;
 }
@@ -4344,9 +4404,14 @@ int slm_hip_linear(slm_hip* c, float* y, const float* w, size_t rows, size_t col
         int64_t ns = nsplit_of((int64_t)cols);
         if (ns > 1) TRY(need_part(c, (size_t)(2 * ns) * rows * 4));
     }
-    if (m > 16) {
+    {
+        // Room for split partials. Few tokens, and columns that are not whole float4s, also run
+        // without (those of more than 256 MB are not asked for).
         int64_t ns = nsplit_of((int64_t)cols);
-        if (ns > 1) TRY(need_gpart(c, (size_t)ns * m * rows * 4));
+        bool vec = cols % 4 == 0 && aligned16(w) && aligned16(x);
+        size_t bytes = (size_t)ns * m * rows * 4;
+        if (ns > 1 && m > SMALL_M && vec) TRY(need_gpart(c, bytes));
+        else if (ns > 1 && bytes <= (size_t)256 << 20) (void)need_gpart(c, bytes);
     }
     Op o = op(OP_LINEAR);
     o.p[0] = y;

@@ -144,3 +144,81 @@ def test_global_layer_input(hip, d, kh, dh, cap, shift, logn, fp16):
     finally:
         hip.set_fusion(True)
         hip.set_fp16(False)
+
+
+# few-token kernels: to 16 and to 32 tokens, tiles of 16, 8 or 4 rows, one launch over the
+# column splits or one a split; past them the GEMMs. Slices of 64 columns, splits of 768;
+# columns that are no multiple of 64 or of 4 (fp32).
+@pytest.mark.parametrize("rows,cols", [(16, 64), (5, 4), (33, 767), (12, 768), (700, 772), (40, 769), (768, 3072),
+                                       (2050, 1536), (31, 2306), (9, 12300)])
+def test_linear_token_ranges(hip, rows, cols):
+    """The same bits for a token whatever the call's other tokens (1, 2, 15 to 18, 31 to 34 and 70
+    of them), from float64 no further than 2e-6 of the largest result (test_gpu_ops.py's bound)."""
+    rng = np.random.default_rng(rows * 10000 + cols)
+    w, x = (rng.standard_normal(s).astype(np.float32) for s in ((rows, cols), (70, cols)))
+    dw, dx, dy = hip.upload(w), hip.upload(x), hip.alloc(70 * rows)
+    hip.linear(dy.ptr, dw.ptr, rows, cols, dx.ptr, 70)
+    want = dy.read().reshape(70, rows)
+    assert rel(want, x.astype(np.float64) @ w.T.astype(np.float64)) < 2e-6
+    for m in (1, 2, 15, 16, 17, 18, 31, 32, 33, 34):
+        hip.upload_into(dy, np.full(70 * rows, np.nan, np.float32))
+        hip.linear(dy.ptr, dw.ptr, rows, cols, dx.at((70 - m) * cols), m)
+        got = dy.read()
+        assert np.array_equal(got[:m * rows].reshape(m, rows), want[70 - m:]), m
+        assert np.isnan(got[m * rows:]).all()
+
+
+@pytest.mark.parametrize("fp16", [False, True])
+@pytest.mark.parametrize("m", [2, 16, 17, 32])
+@pytest.mark.parametrize("kind", ["attention", "linear_attention", "mlp"])
+def test_few_token_epilogues(hip, kind, m, fp16):
+    """The few-token kernels' epilogues (rope and ring stores, per-head L2 norm, the SiLU pair)
+    leave the bits of one launch per operation, ring slots wrapping inside the call."""
+    d, heads, dh, cap, pos = 128, 2, 64, 70, 60
+    rng = np.random.default_rng(m)
+    hip.set_fp16(fp16)
+    try:
+        up = lambda *s: hip.upload(rng.standard_normal(s).astype(np.float32) * np.float32(0.1))  # noqa: E731
+        parts = {"attention": 3, "linear_attention": 4, "mlp": 6}[kind]
+        w, x = up(parts * d, d), up(m, d)
+        inv = hip.upload((1.0 / 10000.0 ** (np.arange(32) / 32)).astype(np.float32))
+        cs, sn = hip.alloc(m * 32), hip.alloc(m * 32)
+        got = []
+        for fuse in (False, True):
+            hip.set_fusion(fuse)
+            o = {n: hip.alloc(m * d * parts) for n in ("y", "col", "q", "k", "v", "g", "out")}
+            ring = [hip.alloc_cache(heads, cap, dh) for _ in range(2)]
+            hip.rope_table(cs.ptr, sn.ptr, inv.ptr, pos, m, 32)
+            hip.linear(o["y"].ptr, w.ptr, parts * d, d, x.ptr, m)
+
+            def col(y, j, n=d):
+                hip.columns(o[y].ptr, o["y"].ptr, m, parts * d, j * n, n)
+
+            if kind == "attention":
+                for j, n in enumerate("qk"):
+                    col("col", j)
+                    hip.rope(o[n].ptr, o["col"].ptr, cs.ptr, sn.ptr, m, heads, dh)
+                col("v", 2)
+                for r, n in zip(ring, "kv"):
+                    hip.store(r.ptr, o[n].ptr, pos, m, cap, heads, dh)
+            elif kind == "linear_attention":
+                for j, n in enumerate("qk"):
+                    col("col", j)
+                    hip.l2norm(o[n].ptr, o["col"].ptr, m * heads, dh)
+                col("v", 2)
+                col("g", 3)
+            else:
+                col("q", 0, 3 * d)
+                col("k", 1, 3 * d)
+                hip.silu_mul(o["out"].ptr, o["q"].ptr, o["k"].ptr, m * 3 * d)
+                for n in "qky":  # (dead after: overwritten)
+                    hip.copy(o[n].ptr, o["v"].ptr, m * d * parts)
+            hip.copy(o["col"].ptr, o["out"].ptr, m * d * parts)
+            hip.flush([t.ptr for t in o.values()] + [r.ptr for r in ring])
+            got.append(([t.read() for t in o.values()] + [r.read() for r in ring], hip.last_plan()["kernels"]))
+        for a, b in zip(got[0][0], got[1][0]):
+            assert np.array_equal(a, b)
+        assert got[1][1] < got[0][1]
+    finally:
+        hip.set_fusion(True)
+        hip.set_fp16(False)
