@@ -142,7 +142,8 @@ struct Kernels {
     // attention input, linear-attention input; plain fp32 for any columns and alignment
     hipFunction_t lin_small[3][2], lin_smalls[3][2], lin_smallr[3][2], lin_smalln[3][2], lin_small1[2];
     hipFunction_t rows;                      // prompt row chains
-    hipFunction_t attn_pq[3];                // prompt attention, superblock shared in LDS
+    hipFunction_t attn_pq[3];                // prompt attention, query tiles sharing copied key tiles
+    hipFunction_t attn_pqs[3], attn_pqs16[3];  // a query tile's segments on four waves
     hipFunction_t gemm2k_32, gemm2k_16;      // 32- and 16-row tiles, two slice groups (fp32)
     hipFunction_t gemm2_48;                  // 48-row tiles, four waves of three row blocks
     hipFunction_t gemm2hk_16, gemm2hwk_16, gemm2h_48, gemm2hw_48;  // the same in fp16 mode
@@ -913,8 +914,17 @@ int lower_one(slm_hip* c, const Op& o, std::vector<Rec>& out) {
                 // a superblock's keys and values pass through LDS for SLM_ATTN_QT query tiles
                 // (then every row's superblocks are combined by a kernel of their own: many
                 // rows, each a wave, rather than one workgroup per tile group at the end)
-                out.push_back(mk(n[9] ? k.attn_pq16[dti] : k.attn_pq[dti], (uint32_t)groups, (uint32_t)kh, (uint32_t)nsb,
-                                 64 * SLM_ATTN_QT, (uint32_t)((SLM_ATTN_NB * 2 + SLM_ATTN_QT) * 16 * 64 * 4),
+                // (the segments on waves of their own, a quarter of the tiles in a wave's chain, while
+                // the query tiles' workgroups with keys to see are few, four a CU: at 576 of
+                // them 21.8 us against 27.0, at 816 25.2 against 28.3, at 960 27.8 against 28.1, at 2700
+                // 45.0 against 39.7)
+                int64_t qt = (m + qpt - 1) / qpt;
+                bool seg = (double)(qt * kh) * o.f[1] <= 4 * CU_COUNT;
+                hipFunction_t pf = seg ? (n[9] ? k.attn_pqs16[dti] : k.attn_pqs[dti]) : n[9] ? k.attn_pq16[dti] : k.attn_pq[dti];
+                uint32_t waves = seg ? SLM_SB_SEGS : SLM_ATTN_QT;
+                uint32_t shmem = seg ? SLM_SB_SEGS * SLM_ATTN_NB * 2 * 16 * 64 * 4 : (SLM_ATTN_NB * 2 + SLM_ATTN_QT) * 16 * 64 * 4;
+                out.push_back(mk(pf, (uint32_t)(seg ? qt : groups), (uint32_t)kh, (uint32_t)nsb,
+                                 64 * waves, shmem,
                                  part, p[1], p[2], p[3], (const long long*)o.dyn, (long long)n[0],
                                  (int)m, (long long)n[2], (long long)n[3], (long long)n[4],
                                  (int)heads, (int)kh, (int)dh, o.f[0]));
@@ -3483,6 +3493,8 @@ int load_kernels(slm_hip* c) {
                {&k.attn[4], "slm_attn_part_16"},
                {&k.attn_dec[0], "slm_attn_dec_1"}, {&k.attn_dec[1], "slm_attn_dec_2"},
                {&k.attn_dec[2], "slm_attn_dec_4"}, {&k.rows, "slm_rows"},
+               {&k.attn_pqs[0], "slm_attn_pqs_1"}, {&k.attn_pqs[1], "slm_attn_pqs_2"}, {&k.attn_pqs[2], "slm_attn_pqs_4"},
+               {&k.attn_pqs16[0], "slm_attn_pqs16_1"}, {&k.attn_pqs16[1], "slm_attn_pqs16_2"}, {&k.attn_pqs16[2], "slm_attn_pqs16_4"},
                {&k.attn_pq[0], "slm_attn_pq_1"}, {&k.attn_pq[1], "slm_attn_pq_2"},
                {&k.attn_pq[2], "slm_attn_pq_4"},     {&k.argmax, "slm_argmax"},
                {&k.gemm2s[0], "slm_gemm2s_32"},   {&k.gemm2s[1], "slm_gemm2s_64"},
@@ -4533,6 +4545,11 @@ int attend_op(slm_hip* c, float* y, const float* q, const float* k, const float*
     o.n[9] = hk ? 1 : 0;
     // the kernels' scores are in powers of two (fp16 mode: the dtype's scalar first, mlx.rs:344)
     o.f[0] = (float)((double)(c->fp16 ? round16(a->scale) : a->scale) * 1.4426950408889634);
+    if (m > 1) {  // superblocks some query sees at this call's position (the grid has nsb slots)
+        size_t first = (size_t)reach - 1 > a->pos ? 0 : a->pos - ((size_t)reach - 1);
+        size_t end = (size_t)gap > a->pos + m ? 0 : a->pos + m - (size_t)gap;
+        o.f[1] = end <= first ? 0.0f : (float)((end - 1) / SLM_SB_KEYS - first / SLM_SB_KEYS + 1);
+    }
     if (hk && m > 1 && (int64_t)((qtiles + SLM_ATTN_QT - 1) / SLM_ATTN_QT) * (int64_t)kh * (int64_t)nsb > (int64_t)INT_MAX)
         return fail(c, SLM_E_UNSUPPORTED, "attend: fp16 rings: %zu query tiles", qtiles);
     return SLM_OK;
