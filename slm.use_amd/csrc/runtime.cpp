@@ -693,7 +693,7 @@ int lower_linear(slm_hip* c, const Op& o, std::vector<Rec>& out, int64_t* fold_n
             }
         };
         bool room = (int64_t)c->gpart_bytes >= ns * m * rows * 4;
-        if (ns == 1 || (!fold_ns && 4 * small_lds(nsl, nv, 16) <= LDS_MAX)) consider(1, 0.0);
+        if (ns == 1 || ((!fold_ns || !room) && 4 * small_lds(nsl, nv, 16) <= LDS_MAX)) consider(1, 0.0);
         if (ns > 1 && room) consider(ns, fold_ns ? 0.0 : 1.7);
         if (best < 0) return fail(c, SLM_E_INVALID, "linear: no room for %lld split partials", (long long)ns);
         int64_t per = z > 1 ? SLM_SPLIT : nsl;
@@ -919,7 +919,7 @@ int lower_one(slm_hip* c, const Op& o, std::vector<Rec>& out) {
                 // them 21.8 us against 27.0, at 816 25.2 against 28.3, at 960 27.8 against 28.1, at 2700
                 // 45.0 against 39.7)
                 int64_t qt = (m + qpt - 1) / qpt;
-                bool seg = (double)(qt * kh) * o.f[1] <= 4 * CU_COUNT;
+                bool seg = (double)(qt * kh) * o.f[1] <= 4 * CU_COUNT && qt * kh * nsb <= (int64_t)INT_MAX;
                 hipFunction_t pf = seg ? (n[9] ? k.attn_pqs16[dti] : k.attn_pqs[dti]) : n[9] ? k.attn_pq16[dti] : k.attn_pq[dti];
                 uint32_t waves = seg ? SLM_SB_SEGS : SLM_ATTN_QT;
                 uint32_t shmem = seg ? SLM_SB_SEGS * SLM_ATTN_NB * 2 * 16 * 64 * 4 : (SLM_ATTN_NB * 2 + SLM_ATTN_QT) * 16 * 64 * 4;
@@ -4417,12 +4417,14 @@ int slm_hip_linear(slm_hip* c, float* y, const float* w, size_t rows, size_t col
         if (ns > 1) TRY(need_part(c, (size_t)(2 * ns) * rows * 4));
     }
     {
-        // Room for split partials. Few tokens, and columns that are not whole float4s, also run
-        // without (those of more than 256 MB are not asked for).
+        // Room for split partials. Few tokens whose partials fit in LDS, and columns that are not
+        // whole float4s, also run without (more than 256 MB are not asked for then).
         int64_t ns = nsplit_of((int64_t)cols);
         bool vec = cols % 4 == 0 && aligned16(w) && aligned16(x);
         size_t bytes = (size_t)ns * m * rows * 4;
-        if (ns > 1 && m > SMALL_M && vec) TRY(need_gpart(c, bytes));
+        int64_t nsl = ((int64_t)cols + 64 - 1) / 64;
+        bool alone = m <= (size_t)SMALL_M ? 4 * small_lds(nsl, small_nv((int64_t)m), 16) <= LDS_MAX : !vec;
+        if (ns > 1 && !alone) TRY(need_gpart(c, bytes));
         else if (ns > 1 && bytes <= (size_t)256 << 20) (void)need_gpart(c, bytes);
     }
     Op o = op(OP_LINEAR);
