@@ -7,8 +7,8 @@
 // in chunks leaves bit-identical state to one read token by token:
 //   - linear: one fixed MFMA chain per output (v_mfma_f32_16x16x4f32 over 16-column
 //     blocks, chained from zero within 64-column slices; slice sums added in order within
-//     768-column splits, split sums added in order); the m <= 16 kernel, the m > 16
-//     kernel and the fused one-token kernel run the same chain;
+//     768-column splits, split sums added in order); the few-token kernels, the prompt
+//     GEMMs and the fused one-token kernel run the same chain;
 //   - attend: keys are grouped by absolute position into 16-key tiles, 64-key segments
 //     and 256-key superblocks; a segment is an online softmax over its tiles, segments
 //     fold into superblocks in order and superblocks into the result in order;
