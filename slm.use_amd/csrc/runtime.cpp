@@ -964,10 +964,12 @@ int lower_one(slm_hip* c, const Op& o, std::vector<Rec>& out) {
 
 struct Range {
     uintptr_t a, b;  // [a, b) bytes
-    bool wg0 = false;  // written by workgroup 0 alone, in program order (a prologue output)
+    bool wg0 = false;   // written by workgroup 0 alone, in program order (a prologue output)
+    bool part = false;  // a write may leave some of it as it was (a cache, an id history)
 };
 Range rng(const float* p, int64_t n) { return Range{(uintptr_t)p, (uintptr_t)(p + n)}; }
 Range rng0(const float* p, int64_t n) { return Range{(uintptr_t)p, (uintptr_t)(p + n), true}; }
+Range rng_part(const float* p, int64_t n) { return Range{(uintptr_t)p, (uintptr_t)(p + n), false, true}; }
 bool overlap(const Range& x, const Range& y) { return x.a < y.b && y.a < x.b; }
 
 // An element-wise one-token op as prologue material: what it reads and writes.
@@ -1961,20 +1963,20 @@ struct Planner {
                 case EPI_SCALE: b.writes.push_back(rng(s.o1, s.rows)); break;
                 case EPI_STORE:
                     for (float* o : {s.o3, s.o4})
-                        if (o) b.writes.push_back(rng(o, ring_floats((int64_t)(s.half / s.dh) * s.cap * s.dh, s.ring16)));
+                        if (o) b.writes.push_back(rng_part(o, ring_floats((int64_t)(s.half / s.dh) * s.cap * s.dh, s.ring16)));
                     break;
                 case EPI_PICK: {
                     const Op& a = ops[i + 1];
                     b.writes.push_back(rng(a.p[0], 2));
-                    if (a.p[2]) b.writes.push_back(rng(a.p[2], a.n[2]));
+                    if (a.p[2]) b.writes.push_back(rng_part(a.p[2], a.n[2]));
                     break;
                 }
                 case EPI_ROPE: {
                     int64_t heads = s.d / s.dh;
                     b.writes.push_back(rng(s.o1, s.d));
                     b.writes.push_back(rng(s.o2, s.d));
-                    b.writes.push_back(rng(s.o3, ring_floats(heads * s.cap * s.dh, s.ring16)));
-                    b.writes.push_back(rng(s.o4, ring_floats(heads * s.cap * s.dh, s.ring16)));
+                    b.writes.push_back(rng_part(s.o3, ring_floats(heads * s.cap * s.dh, s.ring16)));
+                    b.writes.push_back(rng_part(s.o4, ring_floats(heads * s.cap * s.dh, s.ring16)));
                     break;
                 }
             }
@@ -2064,7 +2066,7 @@ struct Planner {
                 if (!o.gout) continue;
                 Range g = rng(o.gout, o.n);
                 bool over = false;  // the epilogue writes all of it (after: the op came before the linear)
-                for (auto& w : b.writes) over = over || (!w.wg0 && w.a <= g.a && g.b <= w.b);
+                for (auto& w : b.writes) over = over || (!w.wg0 && !w.part && w.a <= g.a && g.b <= w.b);
                 if (over || dead_after(ops, i + used, g))
                     o.gout = nullptr;
                 else

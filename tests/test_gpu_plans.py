@@ -1,0 +1,97 @@
+"""One-token op lists whose buffers meet: outputs inside a cache that a later op stores into, in
+place factors, second matrices over what the prologue read. With fusion every buffer holds the bits
+of one launch per operation, and a list takes no more kernels than its parts would.
+"""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+D = 64
+
+
+@pytest.fixture(scope="module")
+def hip(pkg):
+    h = pkg.Hip(0)
+    yield h
+    h.close()
+
+
+class Lists:
+    """Buffers of random values, refilled before each run of a list."""
+
+    def __init__(self, hip):
+        self.hip, self.bufs, self.first = hip, {}, {}
+        self.rng = np.random.default_rng(5)
+        self.inv, self.cs, self.sn = hip.upload(np.ones(D // 2, np.float32)), hip.alloc(D // 2), hip.alloc(D // 2)
+
+    def buf(self, name, n, cache=None):
+        self.bufs[name] = self.hip.alloc_cache(*cache) if cache else self.hip.alloc(n)
+        self.first[name] = self.rng.standard_normal(n).astype(np.float32) * np.float32(0.3)
+
+    def __getitem__(self, name):
+        return self.bufs[name].ptr
+
+    def at(self, name, off):
+        return self.bufs[name].at(off)
+
+    def run(self, ops, fuse, times=1):
+        """Every buffer's bits after `times` runs of the list, and its kernels."""
+        for n, b in self.bufs.items():
+            self.hip.upload_into(b, self.first[n])
+        self.hip.set_fusion(fuse)
+        try:
+            for _ in range(times):
+                self.hip.rope_table(self.cs.ptr, self.sn.ptr, self.inv.ptr, 3, 1, D // 2)
+                ops()
+                self.hip.flush([b.ptr for b in self.bufs.values()])
+            kernels = self.hip.last_plan()["kernels"]
+        finally:
+            self.hip.set_fusion(True)
+        return {n: b.read().view(np.uint32).copy() for n, b in self.bufs.items()}, kernels
+
+    def same(self, ops, most):
+        plain, _ = self.run(ops, False)
+        fused, kernels = self.run(ops, True)
+        for n in plain:
+            assert np.array_equal(plain[n], fused[n]), n
+        assert kernels <= most, kernels
+
+
+@pytest.mark.parametrize("kind", ["store", "rope", "pick"])
+def test_output_inside_a_range_written_in_part(hip, kind):
+    """A copy into another slot of a cache (or another place of an id history) survives the fused
+    store (or pick) that writes one slot (or id) of it."""
+    s = Lists(hip)
+    cap = 8
+    s.buf("x", D), s.buf("n", D), s.buf("g", D), s.buf("row", D), s.buf("w", 3 * D * D), s.buf("y", 3 * D)
+    s.buf("k", cap * D, (1, cap, D)), s.buf("v", cap * D, (1, cap, D))
+    s.buf("q", D), s.buf("kr", D), s.buf("ids", 16), s.buf("tok", 4)
+
+    def ops():
+        h = hip
+        if kind == "pick":
+            h.copy(s.at("ids", 8), s["row"], 4)
+        else:
+            h.copy(s.at("k", 5 * D), s["row"], D)
+        h.rms(s["n"], s["x"], s["g"], 1, D, 1e-6)
+        if kind == "store":
+            h.linear(s["y"], s["w"], 2 * D, D, s["n"], 1)
+            h.store(s["k"], s["y"], 6, 1, cap, 1, D)
+            h.store(s["v"], s.at("y", D), 6, 1, cap, 1, D)
+        elif kind == "rope":
+            h.linear(s["y"], s["w"], 3 * D, D, s["n"], 1)
+            h.rope(s["q"], s["y"], s.cs.ptr, s.sn.ptr, 1, 1, D)
+            h.rope(s["kr"], s.at("y", D), s.cs.ptr, s.sn.ptr, 1, 1, D)
+            h.store(s["k"], s["kr"], 6, 1, cap, 1, D)
+            h.store(s["v"], s.at("y", 2 * D), 6, 1, cap, 1, D)
+        else:
+            h.linear(s["y"], s["w"], 3 * D, D, s["n"], 1)
+            h.argmax(s["tok"], s["ids"], 16, 3, s["y"], 3 * D)
+
+    s.same(ops, 8)
+    got, _ = s.run(ops, True)
+    where = ("ids", 8, 4) if kind == "pick" else ("k", 5 * D, D)
+    assert np.array_equal(got[where[0]][where[1]:where[1] + where[2]],
+                          s.first["row"][:where[2]].view(np.uint32))
