@@ -1052,7 +1052,10 @@ void op_ranges(const Op& o, std::vector<Range>& rd, std::vector<Range>& wr) {
         case OP_GATHER: wr.push_back(rng(p[0], n[0] * n[1])); rd.push_back(rng(p[1], 1)); break;
         case OP_ARGMAX:
             wr.push_back(rng(p[0], 2));
-            if (p[2]) wr.push_back(rng(p[2], n[2]));
+            if (p[2]) {  // (one id of the history: the rest stays, as if read and written back)
+                wr.push_back(rng(p[2], n[2]));
+                rd.push_back(rng(p[2], n[2]));
+            }
             rd.push_back(rng(p[1], n[0]));
             break;
         case OP_COPY: wr.push_back(rng(p[0], n[0])); rd.push_back(rng(p[1], n[0])); break;
@@ -1108,8 +1111,9 @@ void op_ranges(const Op& o, std::vector<Range>& rd, std::vector<Range>& wr) {
             rd.push_back(rng(p[0], ring_floats(n[2] * n[1] * n[3], n[5])));
             rd.push_back(rng(p[1], n[0] * n[2] * n[3]));
             break;
-        case OP_GROW:
+        case OP_GROW:  // (each head's first half)
             wr.push_back(rng(p[0], ring_floats(2 * n[0] * n[1] * n[2], n[3])));
+            rd.push_back(rng(p[0], ring_floats(2 * n[0] * n[1] * n[2], n[3])));
             rd.push_back(rng(p[1], ring_floats(n[0] * n[1] * n[2], n[3])));
             break;
         case OP_ATTEND:

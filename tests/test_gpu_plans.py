@@ -95,3 +95,29 @@ def test_output_inside_a_range_written_in_part(hip, kind):
     where = ("ids", 8, 4) if kind == "pick" else ("k", 5 * D, D)
     assert np.array_equal(got[where[0]][where[1]:where[1] + where[2]],
                           s.first["row"][:where[2]].view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", ["pick", "grow"])
+def test_output_inside_a_range_a_later_op_writes_in_part(hip, kind):
+    """A pick writes one id of its history and a doubling half of each head's slots: what an earlier
+    op put elsewhere in them stays, with other ops between."""
+    s = Lists(hip)
+    s.buf("x", D), s.buf("n", D), s.buf("g", D), s.buf("row", D), s.buf("w", 3 * D * D), s.buf("y", 3 * D)
+    s.buf("y2", D), s.buf("w2", 3 * D * D), s.buf("ids", 16), s.buf("tok", 4)
+    s.buf("k", 4 * D, (1, 4, D)), s.buf("k2", 8 * D, (1, 8, D))
+
+    def ops():
+        if kind == "pick":
+            hip.copy(s.at("ids", 8), s["row"], 4)
+        else:
+            hip.copy(s.at("k2", 6 * D), s["row"], D)
+        hip.rms(s["n"], s["x"], s["g"], 1, D, 1e-6)
+        hip.linear(s["y2"], s["w2"], D, D, s["n"], 1)
+        hip.rms(s["n"], s["y2"], s["g"], 1, D, 1e-6)
+        hip.linear(s["y"], s["w"], 3 * D, D, s["n"], 1)
+        if kind == "pick":
+            hip.argmax(s["tok"], s["ids"], 16, 3, s["y"], 3 * D)
+        else:
+            hip.grow_cache(s.bufs["k2"], s.bufs["k"], 1, 4, D)
+
+    s.same(ops, 6)
