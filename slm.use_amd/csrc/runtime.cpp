@@ -1579,9 +1579,9 @@ struct Planner {
         return row_add(&o, ro, foot);
     }
 
-    // Why a one-token linear runs unfused: printed when SLM_HIP_PLAN_TRACE is set.
+    // Why a one-token linear does not fuse as tried: printed when SLM_HIP_PLAN_TRACE is set.
     size_t nofuse(size_t i, const char* why) {
-        if (c->plan_trace) fprintf(stderr, "slm plan: linear op %zu runs alone: %s\n", i, why);
+        if (c->plan_trace) fprintf(stderr, "slm plan: linear op %zu does not fuse: %s\n", i, why);
         return 0;
     }
 
@@ -1753,8 +1753,18 @@ struct Planner {
     }
 
     // Tries to fuse pend + ops[i] (a one-token linear) + what follows. Returns the number of
-    // ops of `ops` consumed from i (0: no fusion).
+    // ops of `ops` consumed from i (0: no fusion). A group that takes extras (a second matrix, a
+    // factor, stores) and cannot run, their buffers meeting others', is tried again without the
+    // last of them: the rest stays fused.
     size_t try_fg(size_t i) {
+        for (int most = INT_MAX;;) {
+            int extras = 0;
+            size_t used = try_fg(i, most, &extras);
+            if (used || !extras) return used;
+            most = extras - 1;
+        }
+    }
+    size_t try_fg(size_t i, int most, int* extras) {
         const Op& L = ops[i];
         int64_t rows = L.n[0], cols = L.n[1];
         if (L.n[2] != 1 || cols % 16 || cols > VP_LEN_MAX || !aligned16(L.p[1]) || rows < 1 ||
@@ -1839,7 +1849,7 @@ struct Planner {
         }
         // a second matrix on the same input (a global layer's q and kv, model.rs:493-494)
         bool pair = false;
-        if (s0.epi == EPI_PLAIN && nseg == 1 && nsplit == 1 && is(i + 1, OP_LINEAR)) {
+        if (s0.epi == EPI_PLAIN && nseg == 1 && nsplit == 1 && is(i + 1, OP_LINEAR) && *extras < most) {
             const Op& D = ops[i + 1];
             if (D.n[2] == 1 && D.p[2] == x && D.n[1] == cols && D.n[0] >= 1 && D.n[0] <= (int64_t)1 << 26 &&
                 aligned16(D.p[1]) && D.n[3] == L.n[3] && D.n[4] == L.n[4] &&
@@ -1848,6 +1858,7 @@ struct Planner {
                 nseg = 2;
                 used = 2;
                 pair = true;
+                ++*extras;
             }
         }
         // a factor on a matrix's output; stores of parts of one into caches (model.rs:495-528)
@@ -1857,7 +1868,7 @@ struct Planner {
             return -1;
         };
         bool plain = s0.epi == EPI_PLAIN && nsplit == 1 && !hold_q;
-        if (plain && is(i + used, OP_SCALE_ROWS) && ops[i + used].n[0] == 1) {
+        if (plain && is(i + used, OP_SCALE_ROWS) && ops[i + used].n[0] == 1 && *extras < most) {
             const Op& sc = ops[i + used];
             int k = seg_of(sc.p[1], sc.n[1]);
             if (k >= 0 && seg[k].epi == EPI_PLAIN && sc.p[1] == seg[k].y && sc.n[1] == seg[k].rows) {
@@ -1868,9 +1879,10 @@ struct Planner {
                 std::memcpy(&bits, &sc.f[0], 4);
                 seg[k].imm = bits;
                 used++;
+                ++*extras;
             }
         }
-        while (plain && is(i + used, OP_STORE) && ops[i + used].n[0] == 1) {
+        while (plain && is(i + used, OP_STORE) && ops[i + used].n[0] == 1 && *extras < most) {
             const Op& st = ops[i + used];
             int64_t len = st.n[2] * st.n[3];
             int k = seg_of(st.p[1], len);
@@ -1896,6 +1908,7 @@ struct Planner {
                 break;
             }
             used++;
+            ++*extras;
         }
         // MLP up: SiLU of the gate half times the amp half (model.rs:552-555)
         if (s0.epi == EPI_PLAIN && nseg == 1 && nsplit == 1 && is(i + 1, OP_SILU_MUL)) {

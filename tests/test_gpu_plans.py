@@ -121,3 +121,34 @@ def test_output_inside_a_range_a_later_op_writes_in_part(hip, kind):
             hip.grow_cache(s.bufs["k2"], s.bufs["k"], 1, 4, D)
 
     s.same(ops, 6)
+
+
+# kernels: what each list took before matrices were taken in pairs and factors and stores with them
+@pytest.mark.parametrize("kind,most", [("scale in place", 3), ("second over the prologue's input", 2),
+                                       ("two stores into one cache", 3), ("pair and scale in place", 3)])
+def test_lists_with_an_extra_that_cannot_join(hip, kind, most):
+    """An op that cannot join a matrix's launch leaves the matrix fused with what can."""
+    s = Lists(hip)
+    s.buf("x", D), s.buf("n", D), s.buf("g", D), s.buf("y", 2 * D), s.buf("z", D), s.buf("o", D)
+    s.buf("w", 2 * D * D), s.buf("w2", D * D), s.buf("k", 8 * D, (1, 8, D))
+
+    def ops():
+        h = hip
+        h.rms(s["n"], s["x"], s["g"], 1, D, 1e-6)
+        if kind == "scale in place":
+            h.linear(s["z"], s["w2"], D, D, s["n"], 1)
+            h.scale_rows(s["z"], s["z"], np.array([0.37], np.float32), D)
+            h.linear(s["o"], s["w"], D, D, s["z"], 1)
+        elif kind == "second over the prologue's input":
+            h.linear(s["z"], s["w2"], D, D, s["n"], 1)
+            h.linear(s["x"], s["w"], D, D, s["n"], 1)
+        elif kind == "two stores into one cache":
+            h.linear(s["y"], s["w"], 2 * D, D, s["n"], 1)
+            h.store(s["k"], s["y"], 2, 1, 8, 1, D)
+            h.store(s["k"], s.at("y", D), 3, 1, 8, 1, D)
+        else:
+            h.linear(s["z"], s["w2"], D, D, s["n"], 1)
+            h.linear(s["o"], s["w"], D, D, s["n"], 1)
+            h.scale_rows(s["z"], s["z"], np.array([0.37], np.float32), D)
+
+    s.same(ops, most)
