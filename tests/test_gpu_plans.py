@@ -152,3 +152,36 @@ def test_lists_with_an_extra_that_cannot_join(hip, kind, most):
             h.scale_rows(s["z"], s["z"], np.array([0.37], np.float32), D)
 
     s.same(ops, most)
+
+
+@pytest.mark.parametrize("kind,most", [("rope", 2), ("l2norm", 3), ("pick", 2)])
+def test_second_matrix_with_an_epilogue_of_its_own(hip, kind, most):
+    """A matrix whose own launch takes the ops after it (rope and ring stores, the l2norms of a
+    linear-attention input, a pick) is not paired with the matrix before it."""
+    s = Lists(hip)
+    s.buf("x", D), s.buf("n", D), s.buf("g", D), s.buf("a", D), s.buf("wa", D * D), s.buf("w", 4 * D * D)
+    s.buf("y", 4 * D), s.buf("q", D), s.buf("kr", D), s.buf("dec", 4), s.buf("wd", D), s.buf("b", 4)
+    s.buf("k", 8 * D, (1, 8, D)), s.buf("v", 8 * D, (1, 8, D)), s.buf("s", D * D), s.buf("o", D)
+    s.buf("tok", 4), s.buf("ids", 8)
+
+    def ops():
+        h = hip
+        h.rms(s["n"], s["x"], s["g"], 1, D, 1e-6)
+        h.linear(s["a"], s["wa"], D, D, s["n"], 1)
+        if kind == "rope":
+            h.linear(s["y"], s["w"], 3 * D, D, s["n"], 1)
+            h.rope(s["q"], s["y"], s.cs.ptr, s.sn.ptr, 1, 1, D)
+            h.rope(s["kr"], s.at("y", D), s.cs.ptr, s.sn.ptr, 1, 1, D)
+            h.store(s["k"], s["kr"], 6, 1, 8, 1, D)
+            h.store(s["v"], s.at("y", 2 * D), 6, 1, 8, 1, D)
+        elif kind == "l2norm":
+            h.linear(s["y"], s["w"], 4 * D, D, s["n"], 1)
+            h.l2norm(s["q"], s["y"], 1, D)
+            h.l2norm(s["kr"], s.at("y", D), 1, D)
+            h.linear(s["dec"], s["wd"], 1, D, s["n"], 1)
+            h.gla(s["o"], s["s"], s["q"], s["kr"], s.at("y", 2 * D), s["dec"], s["b"], 1, 1, D)
+        else:
+            h.linear(s["y"], s["w"], 3 * D, D, s["n"], 1)
+            h.argmax(s["tok"], s["ids"], 8, 3, s["y"], 3 * D)
+
+    s.same(ops, most)
