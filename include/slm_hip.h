@@ -182,11 +182,15 @@ int slm_hip_attend_noalloc(slm_hip* ctx, float* y, float* scores, const float* q
  * from rope_table to flush — are recorded instead of launched. At flush the planner
  * lowers the step (fusing one-token runs when fusion is on); with graphs on, flush
  * replays a cached hipGraph when the step matches a recorded one (same operations,
- * buffers and sizes; positions, ids and factors may differ) and captures a new one
- * otherwise, and with graphs off it launches the planned kernels directly. A read, free
+ * buffers and sizes; positions, ids and factors may differ): the first run of a step launches
+ * its kernels, the second launches them again and captures the graph behind them; with graphs off it launches the planned kernels directly. A read, free
  * or upload inside a step runs what was recorded so far and finishes the step eagerly.
  * Results are identical in every mode: the same arithmetic runs. */
 int slm_hip_set_graphs(slm_hip* ctx, int on);
+/* Step captures (on by default; no trait counterpart, a test switch): off, the capture of a step
+ * ends without a graph, as when the HIP runtime cannot make one. The step has run by then; its
+ * operations go on being launched kernel by kernel, with the same results. */
+int slm_hip_set_capture(slm_hip* ctx, int on);
 /* One-launch steps (off by default; no trait counterpart, a backend setting): with graphs on,
  * a one-token step whose planned kernels are all fp32 fused GEMVs, one-token attentions that
  * leave their superblock partials to the next fused GEMV and one-token GLAs runs as ONE

@@ -92,6 +92,7 @@ _SIGS = {
     "slm_hip_attend": (_i, [_p, _p, _p, _p, _p, _p, C.POINTER(Attn)]),
     "slm_hip_attend_noalloc": (_i, [_p, _p, _p, _p, _p, _p, C.POINTER(Attn)]),
     "slm_hip_set_graphs": (_i, [_p, _i]),
+    "slm_hip_set_capture": (_i, [_p, _i]),
     "slm_hip_set_step_kernel": (_i, [_p, _i]),
     "slm_hip_step_stats": (_i, [_p, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64), C.POINTER(C.c_int)]),
     "slm_hip_set_prompt_lanes": (_i, [_p, _i]),
@@ -254,6 +255,10 @@ class Hip:
 
     def set_graphs(self, on: bool):
         self.check(lib.slm_hip_set_graphs(self.ctx, int(on)))
+
+    def set_capture(self, on: bool):
+        """Off: step captures end without a graph, as when the runtime cannot make one."""
+        self.check(lib.slm_hip_set_capture(self.ctx, int(on)))
 
     def set_step_kernel(self, on: bool):
         self.check(lib.slm_hip_set_step_kernel(self.ctx, int(on)))

@@ -100,6 +100,7 @@ struct Graph {
     size_t ndyn = 0;
     hipGraphExec_t exec = nullptr;  // null until the step's second run
     std::vector<Rec> recs;          // its planned launches, until then
+    bool launched = false;          // its capture failed: recs are launched each time
     // or, for a one-launch step (slm_step_*): its program in device memory
     char* prog = nullptr;
     int nph = 0, step_var = 0;
@@ -226,6 +227,7 @@ struct slm_hip {
     int* h16_dev = nullptr;              // the code object's mode word slm_h16 (device)
     int fg_rpt = 0;                      // fused GEMV rows per tile: 0 = the planner's choice
     bool timing = false, capturing = false;
+    bool capture_on = true;  // (off: step captures fail, slm_hip_set_capture)
     std::vector<Timed> timed;             // launches whose events are not read yet
     std::vector<hipEvent_t> ev_pool;
     std::map<hipFunction_t, std::string> fname;
@@ -3342,36 +3344,40 @@ int launch_step(slm_hip* c, const Graph& g) {
     return SLM_OK;
 }
 
-// A step's planned launches as a graph, for its next replay.
-int capture_graph(slm_hip* c, Graph& g) {
+// A step's planned launches as a graph, for its next replay. The step itself has been launched by
+// then, so a capture that fails is no error of it: the list goes on being launched kernel by kernel.
+void capture_graph(slm_hip* c, Graph& g) {
     // (nothing is queued here: a read still follows the step before)
     bool armed = c->mir_armed;
     uint64_t last = c->last_graph;
+    std::string err = c->err;
     hipGraph_t graph = nullptr;
-    HIPC(c, hipStreamBeginCapture(mstream(c), hipStreamCaptureModeThreadLocal));
-    c->capturing = true;
-    for (auto& r : g.recs) {
-        int rc = launch_now(c, r);
-        if (rc) {
-            c->capturing = false;
-            hipStreamEndCapture(mstream(c), &graph);
-            if (graph) hipGraphDestroy(graph);
-            return rc;
-        }
+    hipGraphExec_t exec = nullptr;
+    hipStream_t stream = mstream(c);
+    hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
+    if (e == hipSuccess) {
+        c->capturing = true;
+        int rc = SLM_OK;
+        for (auto& r : g.recs)
+            if ((rc = launch_now(c, r))) break;
+        c->capturing = false;
+        e = hipStreamEndCapture(stream, &graph);
+        if (rc) e = hipErrorUnknown;
     }
-    c->capturing = false;
-    HIPC(c, hipStreamEndCapture(mstream(c), &graph));
-    hipError_t e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
-    hipGraphDestroy(graph);
-    if (e != hipSuccess) {
-        g.exec = nullptr;
-        return fail(c, SLM_E_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
+    if (e == hipSuccess) e = c->capture_on ? hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) : hipErrorOutOfMemory;
+    if (graph) hipGraphDestroy(graph);
+    if (e == hipSuccess) {
+        g.exec = exec;
+        std::vector<Rec>().swap(g.recs);
+        c->n_captured++;
+    } else {
+        (void)hipGetLastError();
+        c->err = err;
+        g.launched = true;
+        if (c->plan_trace) fprintf(stderr, "slm graph: a step stays launched: %s\n", hipGetErrorString(e));
     }
-    std::vector<Rec>().swap(g.recs);
-    c->n_captured++;
     c->mir_armed = armed;
     c->last_graph = last;
-    return SLM_OK;
 }
 
 // Runs a recorded step. One-token steps are kept by their op list: the first run of a list plans
@@ -3412,13 +3418,14 @@ int finish_step_run(slm_hip* c) {
         if (g.ops.size() == c->ops.size() && g.ndyn == c->dyn.size() &&
             std::memcmp(g.ops.data(), c->ops.data(), c->ops.size() * sizeof(Op)) == 0) {
             g.used = c->clock;
-            bool second = !g.prog && !g.exec;
+            bool second = !g.prog && !g.exec && !g.launched;
             if (g.prog) TRY(launch_step(c, g));
             else if (g.exec) HIPC(c, hipGraphLaunch(g.exec, mstream(c)));
             else TRY(launch_all(c, g.recs));
             c->n_launched++;
             TRY(after_graph(c, g));
-            return second ? capture_graph(c, g) : SLM_OK;
+            if (second) capture_graph(c, g);
+            return SLM_OK;
         }
     }
     if (c->plan_trace) {  // what sets this step apart from a cached one of the same length
@@ -3951,6 +3958,14 @@ int slm_hip_set_spin_limit(slm_hip* c, long long polls) {
     TRY(taint(c));
     drop_graphs(c);  // the graphs hold the old limit in their descriptors
     c->spin = (int)std::min<long long>(polls, INT_MAX);
+    return SLM_OK;
+}
+
+int slm_hip_set_capture(slm_hip* c, int on) {
+    if (!c) return SLM_E_INVALID;
+    if (c->recording) TRY(finish_step(c));
+    drop_graphs(c);
+    c->capture_on = on != 0;
     return SLM_OK;
 }
 

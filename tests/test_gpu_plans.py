@@ -185,3 +185,33 @@ def test_second_matrix_with_an_epilogue_of_its_own(hip, kind, most):
             h.argmax(s["tok"], s["ids"], 8, 3, s["y"], 3 * D)
 
     s.same(ops, most)
+
+
+def test_step_whose_capture_fails(hip):
+    """A list whose graph cannot be made has run all the same: no error, its state advanced once a
+    run (a running sum, a ring), over replays of another list and after captures work again."""
+    s = Lists(hip)
+    s.buf("x", D), s.buf("n", D), s.buf("g", D), s.buf("w", D * D), s.buf("y", D), s.buf("sum", D)
+    s.buf("k", 8 * D, (1, 8, D))
+
+    def ops():
+        hip.rms(s["n"], s["x"], s["g"], 1, D, 1e-6)
+        hip.linear(s["y"], s["w"], D, D, s["n"], 1)
+        hip.add(s["sum"], s["sum"], s["y"], D)
+        hip.store(s["k"], s["sum"], 3, 1, 8, 1, D)
+
+    want, _ = s.run(ops, True, times=6)
+    hip.set_capture(False)
+    try:
+        before = hip.graph_stats()
+        got, _ = s.run(ops, True, times=6)
+        after = hip.graph_stats()
+    finally:
+        hip.set_capture(True)
+    for n in want:
+        assert np.array_equal(want[n], got[n]), n
+    assert after["captured"] == before["captured"] and after["launched"] == before["launched"] + 6
+    got, _ = s.run(ops, True, times=6)
+    for n in want:
+        assert np.array_equal(want[n], got[n]), n
+    assert hip.graph_stats()["captured"] == after["captured"] + 1
