@@ -697,17 +697,20 @@ int lower_linear(slm_hip* c, const Op& o, std::vector<Rec>& out, int64_t* fold_n
         bool room = (int64_t)c->gpart_bytes >= ns * m * rows * 4;
         if (ns == 1 || ((!fold_ns || !room) && 4 * small_lds(nsl, nv, 16) <= LDS_MAX)) consider(1, 0.0);
         if (ns > 1 && room) consider(ns, fold_ns ? 0.0 : 1.7);
-        if (best < 0) return fail(c, SLM_E_INVALID, "linear: no room for %lld split partials", (long long)ns);
-        int64_t per = z > 1 ? SLM_SPLIT : nsl;
-        out.push_back(mk(vec ? k.lin_small[small_type(o)][nv - 1] : k.lin_small1[nv - 1], (uint32_t)((rows + rt - 1) / rt), 1, (uint32_t)z,
-                         64 * small_waves(per), (uint32_t)(4 * small_lds(per, nv, 16)), p[0], c->gpart, p[1], p[2],
-                         (int)rows, (int)cols, (int)m, rt));
-        out.back().abytes = ab;
-        if (fold_ns) *fold_ns = z;
-        else if (z > 1)
-            out.push_back(mk(k.fold, blocks_for(m * rows), 1, 1, 256, 0, p[0],
-                             (const float*)c->gpart, (long long)(m * rows), (int)z));
-        return SLM_OK;
+        // (no room, and partials past LDS: columns that are not whole float4s go to slm_gemm_s below)
+        if (best < 0 && vec) return fail(c, SLM_E_INVALID, "linear: no room for %lld split partials", (long long)ns);
+        if (best >= 0) {
+            int64_t per = z > 1 ? SLM_SPLIT : nsl;
+            out.push_back(mk(vec ? k.lin_small[small_type(o)][nv - 1] : k.lin_small1[nv - 1], (uint32_t)((rows + rt - 1) / rt), 1, (uint32_t)z,
+                             64 * small_waves(per), (uint32_t)(4 * small_lds(per, nv, 16)), p[0], c->gpart, p[1], p[2],
+                             (int)rows, (int)cols, (int)m, rt));
+            out.back().abytes = ab;
+            if (fold_ns) *fold_ns = z;
+            else if (z > 1)
+                out.push_back(mk(k.fold, blocks_for(m * rows), 1, 1, 256, 0, p[0],
+                                 (const float*)c->gpart, (long long)(m * rows), (int)z));
+            return SLM_OK;
+        }
     }
     {  // the LDS-staged GEMMs, one workgroup column per split
         int64_t ns = (nsl + SLM_SPLIT - 1) / SLM_SPLIT;
@@ -2879,6 +2882,20 @@ int need_gpart(slm_hip* c, size_t bytes) {
     return SLM_OK;
 }
 
+// Room a linear can run without: not asked for while a caller captures the stream (an allocation
+// would end the capture), and not missed where there is none left.
+void offer_gpart(slm_hip* c, size_t bytes) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (bytes <= c->gpart_bytes || hipStreamIsCapturing(c->stream, &st) != hipSuccess ||
+        st != hipStreamCaptureStatusNone)
+        return;
+    std::string err = c->err;
+    if (need_gpart(c, bytes)) {
+        (void)hipGetLastError();
+        c->err = err;
+    }
+}
+
 int need_ws(slm_hip* c, size_t bytes) {
     bytes += 64;  // fused prologues read whole float4s past an odd-sized end
     if (bytes <= c->ws_bytes) return SLM_OK;
@@ -4461,9 +4478,9 @@ int slm_hip_linear(slm_hip* c, float* y, const float* w, size_t rows, size_t col
         bool vec = cols % 4 == 0 && aligned16(w) && aligned16(x);
         size_t bytes = (size_t)ns * m * rows * 4;
         int64_t nsl = ((int64_t)cols + 64 - 1) / 64;
-        bool alone = m <= (size_t)SMALL_M ? 4 * small_lds(nsl, small_nv((int64_t)m), 16) <= LDS_MAX : !vec;
+        bool alone = !vec || (m <= (size_t)SMALL_M && 4 * small_lds(nsl, small_nv((int64_t)m), 16) <= LDS_MAX);
         if (ns > 1 && !alone) TRY(need_gpart(c, bytes));
-        else if (ns > 1 && bytes <= (size_t)256 << 20) (void)need_gpart(c, bytes);
+        else if (ns > 1 && bytes <= (size_t)256 << 20) offer_gpart(c, bytes);
     }
     Op o = op(OP_LINEAR);
     o.p[0] = y;

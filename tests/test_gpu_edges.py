@@ -4,6 +4,8 @@ References are the oracle or float64; every multi-token result is also compared 
 with the same tokens taken one at a time or a few at a time.
 """
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -222,3 +224,37 @@ def test_few_token_epilogues(hip, kind, m, fp16):
     finally:
         hip.set_fusion(True)
         hip.set_fp16(False)
+
+
+# the first linear of a context under a caller's capture: split partials that fit in LDS, some that
+# would take more than a pooled block, and columns that are no whole float4s past what LDS holds
+@pytest.mark.parametrize("rows,cols,m", [(96, 3072, 5), (88000, 4096, 16), (40, 12301, 16)])
+def test_linear_under_a_callers_capture(pkg, rows, cols, m):
+    """No allocation: the capture ends with a graph, whose replays give the eager call's bits."""
+    rng = np.random.default_rng(rows)
+    hip, rt = pkg.Hip(0), pkg.lib
+    try:
+        w, some = hip.alloc(rows * cols), min(rows, 64)
+        for r in (0, rows - some):
+            hip.upload_into(w, rng.standard_normal(some * cols).astype(np.float32), r * cols)
+        x, y, nan = hip.upload(rng.standard_normal(m * cols).astype(np.float32)), hip.alloc(m * rows), np.full(m * rows, np.nan, np.float32)
+        stream, graph, run = C.c_void_p(hip.stream()), C.c_void_p(), C.c_void_p()
+        y.read()
+        assert rt.hipStreamBeginCapture(stream, 1) == 0
+        hip.linear(y.ptr, w.ptr, rows, cols, x.ptr, m)
+        assert rt.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert rt.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+        got = []
+        for _ in range(3):
+            hip.upload_into(y, nan)
+            assert rt.hipGraphLaunch(run, stream) == 0
+            got.append(y.read())
+        rt.hipGraphExecDestroy(run), rt.hipGraphDestroy(graph)
+        hip.upload_into(y, nan)
+        hip.linear(y.ptr, w.ptr, rows, cols, x.ptr, m)
+        want = y.read()
+        assert np.isfinite(want).all() and np.abs(want).max() > 1
+        for g in got:
+            assert np.array_equal(g, want)
+    finally:
+        hip.close()
