@@ -1439,8 +1439,8 @@ __device__ void gemm2_body(float* __restrict__ y, float* __restrict__ part,
 // partials meet in LDS and one pass adds them in order. What bounds these shapes is latency, not
 // rate: the prompt GEMMs below walk a split's twelve slices one after another through LDS, a
 // memory round trip each (a 21-token 2304 x 768 projection 20 us); here all twelve are in
-// flight together. Each workgroup reads all its tokens, so past 32 tokens the GEMMs, whose tiles
-// share them, are the faster. 768 x 3072 at 5 tokens 13.8 -> 7.4 us (with the launch that adds its
+// flight together. Each workgroup reads all its tokens, so the GEMMs, whose tiles share
+// them, are the faster past 32 tokens and, for many rows, past 16 (few_tokens in runtime.cpp). 768 x 3072 at 5 tokens 13.8 -> 7.4 us (with the launch that adds its
 // four splits), 2304 x 768 5.3 -> 4.3; 2304 x 768 with the attention epilogue at 21 tokens 20 -> 7.
 // EPI 0: y [m][rows] (or, with several splits in blockIdx.z, part[split][m][rows]); rt rows a
 // tile (16, 8 or 4: a short matrix spreads over more CUs; the other MFMA rows are zeros).

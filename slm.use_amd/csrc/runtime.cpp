@@ -609,15 +609,18 @@ void drop_graphs(slm_hip* c) {
 // The pipelined prompt GEMM's row tile: the one that leaves the busiest CU the least work —
 // rows per tile times the workgroups a CU runs (32-row tiles of four waves go two to a CU,
 // the others one) — the larger tile on a tie.
+int64_t gemm2_work(int64_t t, int64_t rows, int64_t m, int64_t ns) {
+    int64_t wgs = ((rows + t - 1) / t) * ((m + 63) / 64) * ns;
+    int64_t per_cu = t == 32 ? 2 : 1;
+    int64_t rounds = (wgs + per_cu * CU_COUNT - 1) / (per_cu * CU_COUNT);
+    int64_t sharing = std::min<int64_t>(per_cu, (wgs + CU_COUNT - 1) / CU_COUNT);
+    return rounds * t * sharing;
+}
 int gemm2_bm(int64_t rows, int64_t m, int64_t ns) {
     int bm = 32;
     int64_t best = -1;
     for (int t : {32, 64, 96, 128}) {
-        int64_t wgs = ((rows + t - 1) / t) * ((m + 63) / 64) * ns;
-        int64_t per_cu = t == 32 ? 2 : 1;
-        int64_t rounds = (wgs + per_cu * CU_COUNT - 1) / (per_cu * CU_COUNT);
-        int64_t sharing = std::min<int64_t>(per_cu, (wgs + CU_COUNT - 1) / CU_COUNT);
-        int64_t cost = rounds * t * sharing;
+        int64_t cost = gemm2_work(t, rows, m, ns);
         if (best < 0 || cost <= best) best = cost, bm = t;
     }
     return bm;
@@ -641,16 +644,59 @@ int gemm2_bm_plain(int64_t rows, int64_t m, int64_t ns) {
     return bm;
 }
 
-// The few-token kernels (slm_linear_small*), up to SMALL_M tokens. Every workgroup reads all the
-// tokens, so their time grows with them: 2304 x 768 took 4.3 us at 5 tokens, 6.6 at 32, 8.7 at 48,
-// 10.7 at 64, the GEMMs, which walk the columns through LDS, 7.7 to 7.9 from 17 to 64 (6144 x 768:
-// 7.0, 11.9, 15.7, 19.0 against 11.2 to 11.5).
+// The few-token kernels (slm_linear_small*) take up to SMALL_M tokens; few_tokens() says where they are
+// the faster.
 constexpr int64_t SMALL_M = 32;
 int small_nv(int64_t m) { return (int)((std::min<int64_t>(m, SMALL_M) + 15) / 16); }  // 16-token blocks
 int small_type(const Op& L) { return L.n[4] ? 2 : L.n[3] ? 1 : 0; }
 // LDS floats of `slices` slice partials and the epilogue's tile, `tr` tile rows
 int64_t small_lds(int64_t slices, int nv, int tr) { return slices * 16 * nv * tr + 16 * nv * (tr + 1); }
 uint32_t small_waves(int64_t slices) { return (uint32_t)std::min<int64_t>(slices, 16); }
+
+// Of `tiles` workgroups a split of SLM_SPLIT slices (the last split the rest), the splits one after
+// another, CU_COUNT workgroups at a time: the 64-column slices the busiest CU runs, and its workgroups.
+int64_t cu_slices(int64_t tiles, int64_t nsl, int64_t* wgs) {
+    int64_t ns = (nsl + SLM_SPLIT - 1) / SLM_SPLIT;
+    int64_t full = (tiles * (ns - 1) + CU_COUNT - 1) / CU_COUNT;
+    *wgs = (tiles * ns + CU_COUNT - 1) / CU_COUNT;
+    return full * SLM_SPLIT + (*wgs - full) * (nsl - (ns - 1) * SLM_SPLIT);
+}
+
+// Which kernels a linear of m tokens takes: the few-token ones to 16 tokens; from 17 to SMALL_M
+// the shorter of the two times estimated here, in us. Every few-token workgroup reads all the
+// tokens, so its time grows with them and with the workgroups a CU runs in turn; the GEMMs' tiles of
+// 64 tokens take the same time from 17 to 64. Measured at 17 and 32 tokens, few-token
+// kernel against GEMM: fp32 2304 x 768 6.1 and 6.5 against 7.7, 6144 x 768 10.3 and 11.8 against
+// 11.2, 32000 x 768 38 and 45 against 33, 4096 x 4096 26 and 29 against 37; fp16 2304 x 768 5.5 and 6.4
+// against 5.9, 6144 x 768 9.3 and 11.1 against 8.9, 32000 x 768 34 and 41 against 14; up projection's
+// epilogue, 6144 x 768, 11.8 and 12.1 against 11.0 and 9.9, fp16 10.2 and 11.4 against 7.1 and
+// 6.6; attention input, 2304 x 768, 7.3 and 8.2 against 18, fp16 7.3 and 8.0 against 8.8; linear-attention
+// input, 3072 x 768, 16.9 and 19.9 against 18, fp16 15.2 and 19.4 against 8.8. Over 127 shapes of
+// 256 to 32000 rows and 128 to 4096 columns the rule's choice takes 0.6 % longer than the better kernel.
+enum { LIN_PLAIN, LIN_SILU, LIN_ROPE, LIN_NORM };
+bool few_tokens(int64_t rows, int64_t cols, int64_t m, bool h, int kind, bool vec = true) {
+    if (m <= 16 || m > SMALL_M) return m <= 16;
+    int64_t nsl = (cols + 63) / 64, ns = (nsl + SLM_SPLIT - 1) / SLM_SPLIT;
+    auto tiles = [&](int64_t t) { return (rows + t - 1) / t; };
+    if (kind == LIN_NORM) return !h && m <= 20 && nsl >= 8;  // (a head of 64 rows a workgroup)
+    int64_t wgs, gwgs;
+    double load = (double)cu_slices(tiles(16), nsl, &wgs);
+    double small = 2.5 + load * (h ? 0.185 + 0.0055 * (double)m : 0.26 + 0.004 * (double)m) + 0.1 * (double)(wgs - 1);
+    if (kind != LIN_PLAIN) {
+        int64_t work = 64 * ((tiles(64) + CU_COUNT - 1) / CU_COUNT);  // tile rows a CU runs
+        if (kind == LIN_SILU) work = gemm2_work(gemm2_bm(rows, m, 1), rows, m, 1);
+        return small + 0.2 < (h ? 3.2 + 0.0075 * (double)(nsl * work) : 1.6 + 0.0216 * (double)(nsl * work));
+    }
+    if (!vec || cols % 64) {  // (slm_gemm, slm_gemm_s)
+        if (!vec) small = 1.2 + load * (0.69 + 0.0153 * (double)m);
+        return small < 3.7 + (vec ? 1.5 : 2.5) * (double)cu_slices(tiles(64), nsl, &gwgs);
+    }
+    int64_t bm = gemm2_bm_plain(rows, m, ns);
+    if (bm == 32 && h) bm = 48;
+    double gload = (double)cu_slices(tiles(bm), nsl, &gwgs);
+    double gemm = h ? 3.9 + 0.0067 * gload * ((double)bm + 14) : 3.0 * (double)gwgs + 0.0196 * gload * ((double)bm + 3.6);
+    return small < gemm + (ns == 1 ? 0.0 : h ? 0.5 : 1.0);
+}
 
 // A linear (p0 y, p1 w, p2 x; n0 rows, n1 cols, n2 m). With `fold_ns`, a split GEMM's
 // partials are left in c->gpart for the caller to add (*fold_ns: the split count, 1 when
@@ -675,9 +721,10 @@ int lower_linear(slm_hip* c, const Op& o, std::vector<Rec>& out, int64_t* fold_n
     if (h && (!vec || cols % 64 || (m <= 16 && nsl > 64)))
         return fail(c, SLM_E_UNSUPPORTED, "linear: fp16 mode has no kernel for %lld x %lld x %lld",
                     (long long)rows, (long long)cols, (long long)m);
-    if (m <= SMALL_M) {
+    int64_t ns = (nsl + SLM_SPLIT - 1) / SLM_SPLIT;
+    bool room = ns == 1 || (int64_t)c->gpart_bytes >= ns * m * rows * 4;  // for split partials
+    if (m <= SMALL_M && (!room || few_tokens(rows, cols, m, h, LIN_PLAIN, vec))) {
         int nv = small_nv(m);
-        int64_t ns = (nsl + SLM_SPLIT - 1) / SLM_SPLIT;
         // one launch over all the splits where their partials fit in LDS, or a split in each
         // blockIdx.z (always where the caller adds the partials). The busiest CU's time, us: its
         // weights and tokens at 50 KB/us, its MFMAs (sixteen rows whatever the tile holds), and
@@ -694,7 +741,6 @@ int lower_linear(slm_hip* c, const Op& o, std::vector<Rec>& out, int64_t* fold_n
                 if (best < 0 || us < (t == 16 ? best : 0.9 * best)) best = us, rt = t, z = zs;
             }
         };
-        bool room = (int64_t)c->gpart_bytes >= ns * m * rows * 4;
         if (ns == 1 || ((!fold_ns || !room) && 4 * small_lds(nsl, nv, 16) <= LDS_MAX)) consider(1, 0.0);
         if (ns > 1 && room) consider(ns, fold_ns ? 0.0 : 1.7);
         // (no room, and partials past LDS: columns that are not whole float4s go to slm_gemm_s below)
@@ -713,8 +759,6 @@ int lower_linear(slm_hip* c, const Op& o, std::vector<Rec>& out, int64_t* fold_n
         }
     }
     {  // the LDS-staged GEMMs, one workgroup column per split
-        int64_t ns = (nsl + SLM_SPLIT - 1) / SLM_SPLIT;
-        bool room = ns == 1 || (int64_t)c->gpart_bytes >= ns * m * rows * 4;
         if (!room && vec) return fail(c, SLM_E_INVALID, "linear: no room for %lld split partials", (long long)ns);
         if (!room) ns = 1;  // (slm_gemm_s then adds its splits itself)
         if (vec && cols % 64 == 0) {
@@ -2291,7 +2335,7 @@ struct Planner {
             return 0;
         Range ry = rng(sm.p[0], m * h);
         if (overlap(ry, rng(L.p[1], wfloats(L))) || overlap(ry, rng(L.p[2], m * cols))) return 0;
-        if (m <= SMALL_M) {
+        if (few_tokens(rows, cols, m, L.n[3] != 0, LIN_SILU)) {
             int nv = small_nv(m);
             out.push_back(mk(c->k.lin_smalls[small_type(L)][nv - 1], (uint32_t)((h + 7) / 8), 1, 1, 64 * small_waves(cols / 64),
                              (uint32_t)(4 * small_lds(cols / 64, nv, 16)), sm.p[0], c->gpart, L.p[1], L.p[2],
@@ -2361,7 +2405,7 @@ struct Planner {
                 if (overlap(wr[a], x)) return 0;
         }
         if (!dead_after(ops, i + 8, rng(cy, m * d))) return 0;
-        bool few = m <= SMALL_M;
+        bool few = few_tokens(rows, cols, m, L.n[3] != 0, LIN_ROPE);
         int nv = small_nv(m);
         uint32_t shmem = few ? (uint32_t)(4 * small_lds(cols / 64, nv, 16))
                              : (uint32_t)(GEMM_STAGES_HOST * (64 * (L.n[4] ? 32 : 64) + 64 * 64) * 4);
@@ -2413,7 +2457,7 @@ struct Planner {
                 if (overlap(wr[a], x)) return 0;
         }
         if (!dead_after(ops, i + 7, rng(cy, m * d))) return 0;
-        bool few = m <= SMALL_M;
+        bool few = few_tokens(rows, cols, m, L.n[3] != 0, LIN_NORM);
         int nv = small_nv(m);
         uint32_t shmem = few ? (uint32_t)(4 * small_lds(cols / 64, nv, 64))
                              : (uint32_t)(GEMM_STAGES_HOST * (64 * (L.n[4] ? 32 : 64) + 64 * 64) * 4);

@@ -170,6 +170,41 @@ def test_linear_token_ranges(hip, rows, cols):
         assert np.isnan(got[m * rows:]).all()
 
 
+# either side of the rule for 17 to 32 tokens (few-token kernels or GEMMs): plain linears
+@pytest.mark.parametrize("rows,cols,m,fp16,few", [
+    (2304, 768, 17, False, True), (2304, 768, 32, False, True), (32000, 768, 17, False, False),
+    (4096, 1536, 24, False, True), (3072, 3072, 32, False, False), (768, 3072, 32, False, True),
+    (512, 768, 17, True, True), (6144, 768, 32, True, False), (32000, 768, 20, True, False),
+    (4096, 1024, 32, True, True), (3072, 3072, 17, True, False), (96, 770, 32, False, True),
+    (12288, 770, 32, False, False), (32000, 772, 32, False, False), (32000, 768, 16, True, True)])
+def test_linear_17_to_32_tokens(hip, rows, cols, m, fp16, few):
+    """The kernels the rule names run, and leave the bits of 1 and m - 1 tokens in calls of their own
+    and of a 40-token call."""
+    rng = np.random.default_rng(rows + m)
+    hip.set_fp16(fp16)
+    try:
+        w = hip.upload((rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+        x, y = hip.upload(rng.standard_normal((40, cols)).astype(np.float32)), hip.alloc(40 * rows)
+        hip.linear(y.ptr, w.ptr, rows, cols, x.ptr, 40)
+        want = y.read()[:m * rows]
+        hip.linear(y.ptr, w.ptr, rows, cols, x.ptr, 1)
+        hip.linear(y.at(rows), w.ptr, rows, cols, x.at(cols), m - 1)
+        assert np.array_equal(y.read()[:m * rows], want)
+        hip.upload_into(y, np.full(40 * rows, np.nan, np.float32))
+        hip.set_timing(True)
+        hip.linear(y.ptr, w.ptr, rows, cols, x.ptr, m)
+        got = y.read()
+        assert np.array_equal(got[:m * rows], want) and np.isnan(got[m * rows:]).all()
+        kind = "s" if cols % 4 else "v" + ("hw" if fp16 else "")
+        ran = hip.kernel_stat(f"slm_linear_small_{kind}_{(m + 15) // 16}")["launches"]
+        assert ran == int(few)
+    finally:
+        hip.set_timing(False)
+        hip.set_fp16(False)
+        for b in (w, x, y):
+            b.free()
+
+
 @pytest.mark.parametrize("fp16", [False, True])
 @pytest.mark.parametrize("m", [2, 16, 17, 32])
 @pytest.mark.parametrize("kind", ["attention", "linear_attention", "mlp"])
