@@ -91,6 +91,25 @@ def test_attend_tiles(hip, pos, m, reach, gap, cap, heads, kh, dh):
     assert rel(got.ravel(), exact) <= 2 * rel(want, exact) + 1e-7
 
 
+# one token, a query tile's segments on waves of their own, query tiles sharing key tiles, the general kernel
+@pytest.mark.parametrize("m,heads,dh", [(1, 2, 64), (3, 2, 64), (256, 12, 64), (40, 1, 32), (5, 1, 128), (1, 1, 128)])
+def test_attend_weights_of_large_scores(hip, m, heads, dh):
+    """Scores near +-100, exact in 32 bits, 0 to 4 under their maximum: a weight's exponent is at most 5.8
+    in powers of two, off by half its last step (1.7e-7 of the weight) and the exponential's ulp
+    (1.2e-7), whatever the scores' own size; with sums and values 5e-7 of the largest result."""
+    rng = np.random.default_rng(dh + m)
+    n = 4096
+    q, k = np.zeros((m, heads, dh), np.float32), np.zeros((heads, n, dh), np.float32)
+    q[:, :, 0] = 1.0
+    k[:, :, 0] = rng.choice([-800.0, 800.0], (heads, 1)) - np.round(rng.random((heads, n)) * 32 * 512) / 512
+    v = rng.standard_normal((heads, n, dh)).astype(np.float32)
+    a = dict(pos=n - m, m=m, reach=O.USIZE_MAX, gap=0, cap=n, heads=heads, key_heads=heads, dh=dh, scale=0.125)
+    dq, dk, dv, dy = hip.upload(q), hip.upload(k), hip.upload(v), hip.alloc(q.size)
+    hip.attend(dy.ptr, dq.ptr, dk.ptr, dv.ptr, **a)
+    err = rel(dy.read(), attend64(q, k, v, **a))
+    assert err < 5e-7
+
+
 @pytest.mark.parametrize("fp16", [False, True])
 @pytest.mark.parametrize("d,kh,dh,cap,shift,logn", [(768, 4, 64, 300, True, True), (768, 4, 64, 128, False, True),
                                                     (64, 1, 16, 64, True, False), (128, 2, 48, 65, False, False)])
