@@ -2315,9 +2315,7 @@ __device__ __forceinline__ void attn_pq_run(float* __restrict__ part, const floa
     }
     auto where = [&](int t, int n) {
         unsigned slot = base + (unsigned)(16 * t + 4 * (row0 + SHARE * n) + g);
-        if (wrap1) slot = slot >= cap32 ? slot - cap32 : slot;
-        else
-            while (slot >= cap32) slot -= cap32;
+        slot = wrap1 ? (slot >= cap32 ? slot - cap32 : slot) : slot % cap32;
         return (long long)slot * dh + 4 * chunk[n];
     };
     const float *kb = kc + (long long)kvh * cap * dh, *vb = vc + (long long)kvh * cap * dh;

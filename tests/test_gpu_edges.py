@@ -65,8 +65,8 @@ def test_gla_blocks(hip, m, heads, dh, fp16):
         hip.set_fp16(False)
 
 
-# four query tiles of 16 / group queries a workgroup; 16-key tiles, 64-key segments, 256-key
-# superblocks; rings shorter than a superblock, spans that start or end inside a tile
+# a query tile of 16 / group queries a workgroup, its segments on four waves (calls this short: longer
+# ones are in test_attend_shared_tiles); 16-key tiles, 64-key segments, 256-key superblocks; rings shorter than a superblock, spans that start or end inside a tile
 @pytest.mark.parametrize("pos,m,reach,gap,cap,heads,kh,dh", [
     (0, 2, O.USIZE_MAX, 0, 300, 2, 2, 64), (0, 64, O.USIZE_MAX, 0, 64, 1, 1, 64), (1000, 65, 100, 0, 165, 2, 2, 64),
     (255, 17, 256, 0, 512, 1, 1, 64), (513, 63, 49, 0, 112, 2, 1, 60), (300, 33, O.USIZE_MAX, 64, 400, 8, 1, 64),
@@ -89,6 +89,48 @@ def test_attend_tiles(hip, pos, m, reach, gap, cap, heads, kh, dh):
         assert np.array_equal(d1.read(), got[i]), i
     want, exact = O.attend(q, k, v, **a), attend64(q, k, v, **a)
     assert rel(got.ravel(), exact) <= 2 * rel(want, exact) + 1e-7
+
+
+# calls past the 1024 (query tiles x key heads x visible superblocks) from which query tiles share
+# copied key tiles: head sizes in 1, 2 and 4 blocks of 16 and between them, 1 to 4 heads a key head, a
+# gap, a ragged last group of tiles, rings shorter than a superblock
+SHARED = [
+    (5000, 300, 4096, 0, 4400, 12, 12, 64), (3000, 403, O.USIZE_MAX, 64, 3500, 3, 1, 60), (0, 3001, 150, 0, 200, 2, 2, 48),
+    (700, 1030, 512, 100, 1600, 8, 2, 32), (30, 2500, 5, 0, 5, 1, 1, 24), (2000, 777, 1000, 0, 1777, 4, 4, 16),
+    (2000, 777, 1000, 0, 900, 4, 4, 8)]
+
+
+# (fp16 mode: the rings that it keeps in fp16)
+@pytest.mark.parametrize("pos,m,reach,gap,cap,heads,kh,dh,fp16", [
+    (*c, f) for c in SHARED for f in (False, True) if not f or (c[7] % 8 == 0 and c[4] >= 64)])
+def test_attend_shared_tiles(hip, pos, m, reach, gap, cap, heads, kh, dh, fp16):
+    """Against float64 (fp32: no further than twice the oracle's sums; fp16 mode: half a step of its
+    rounding), and the bits of queries taken alone: the first, the last and some between."""
+    rng = np.random.default_rng(pos + m + dh)
+    a = dict(pos=pos, m=m, reach=reach, gap=gap, cap=cap, heads=heads, key_heads=kh, dh=dh, scale=0.25)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((m, heads, dh), (kh, cap, dh), (kh, cap, dh)))
+    dt = 1 if dh <= 16 else 2 if dh <= 32 else 4
+    hip.set_fp16(fp16)
+    try:
+        if fp16:
+            q, k, v = (t.astype(np.float16).astype(np.float32) for t in (q, k, v))
+        dk, dv = hip.alloc_cache(kh, cap, dh), hip.alloc_cache(kh, cap, dh)
+        hip.upload_into(dk, k), hip.upload_into(dv, v)
+        dq, dy, d1 = hip.upload(q), hip.alloc(q.size), hip.alloc(heads * dh)
+        hip.set_timing(True)
+        hip.attend(dy.ptr, dq.ptr, dk.ptr, dv.ptr, **a)
+        got = dy.read().reshape(m, -1)
+        assert hip.kernel_stat(f"slm_attn_pq{'16' if fp16 else ''}_{dt}")["launches"] == 1
+        hip.set_timing(False)
+        for i in sorted({0, 1, m - 2, m - 1, *range(15, m, max(1, m // 40))}):
+            hip.attend(d1.ptr, dq.at(i * heads * dh), dk.ptr, dv.ptr, **dict(a, pos=pos + i, m=1))
+            assert np.array_equal(d1.read(), got[i]), i
+    finally:
+        hip.set_timing(False)
+        hip.set_fp16(False)
+    exact = attend64(q, k, v, **a)
+    err = rel(got.ravel(), exact)
+    assert err <= (2.0 ** -11 + 2e-6 if fp16 else 2 * rel(O.attend(q, k, v, **a), exact) + 1e-7)
 
 
 # one token, a query tile's segments on waves of their own, query tiles sharing key tiles, the general kernel
