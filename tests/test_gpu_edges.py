@@ -66,7 +66,8 @@ def test_gla_blocks(hip, m, heads, dh, fp16):
 
 
 # a query tile of 16 / group queries a workgroup, its segments on four waves (calls this short: longer
-# ones are in test_attend_shared_tiles); 16-key tiles, 64-key segments, 256-key superblocks; rings shorter than a superblock, spans that start or end inside a tile
+# ones are in test_attend_shared_tiles); 16-key tiles, 64-key segments, 256-key superblocks; rings
+# shorter than a superblock, spans that start or end inside a tile
 @pytest.mark.parametrize("pos,m,reach,gap,cap,heads,kh,dh", [
     (0, 2, O.USIZE_MAX, 0, 300, 2, 2, 64), (0, 64, O.USIZE_MAX, 0, 64, 1, 1, 64), (1000, 65, 100, 0, 165, 2, 2, 64),
     (255, 17, 256, 0, 512, 1, 1, 64), (513, 63, 49, 0, 112, 2, 1, 60), (300, 33, O.USIZE_MAX, 64, 400, 8, 1, 64),
@@ -133,6 +134,43 @@ def test_attend_shared_tiles(hip, pos, m, reach, gap, cap, heads, kh, dh, fp16):
     assert err <= (2.0 ** -11 + 2e-6 if fp16 else 2 * rel(O.attend(q, k, v, **a), exact) + 1e-7)
 
 
+# a visible key or value that is infinite or NaN, in every attention kernel (one superblock)
+@pytest.mark.parametrize("m,heads,dh,n", [(1, 2, 64, 250), (3, 2, 64, 250), (100, 160, 64, 250), (5, 2, 128, 250), (1, 2, 128, 250)])
+@pytest.mark.parametrize("what", ["k nan", "k inf", "k -inf", "v inf", "v nan"])
+def test_attend_visible_infinities(hip, m, heads, dh, n, what):
+    """A score of -inf weighs nothing; a value's infinity or NaN reaches its own dim only; a score of
+    +inf or NaN leaves its superblock out. The other heads are untouched."""
+    rng = np.random.default_rng(n + m)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((m, heads, dh), (heads, n, dh), (heads, n, dh)))
+    q[:, :, 0] = np.abs(q[:, :, 0]) + 0.5  # (an infinite key coordinate gives an infinite score of its sign)
+    a = dict(pos=n - m, m=m, reach=O.USIZE_MAX, gap=0, cap=n, heads=heads, key_heads=heads, dh=dh, scale=0.125)
+    dq, dk, dv, dy = hip.upload(q), hip.upload(k), hip.upload(v), hip.alloc(q.size)
+    hip.attend(dy.ptr, dq.ptr, dk.ptr, dv.ptr, **a)
+    plain = dy.read().reshape(m, heads, dh)
+    at, val = 70, {"nan": np.nan, "inf": np.inf, "-inf": -np.inf}[what[2:]]
+    (k if what[0] == "k" else v)[0, at, 0 if what[0] == "k" else 3] = val
+    hip.upload_into(dk, k), hip.upload_into(dv, v)
+    hip.attend(dy.ptr, dq.ptr, dk.ptr, dv.ptr, **a)
+    got = dy.read().reshape(m, heads, dh)
+    same = np.array_equal(got[:, 1:], plain[:, 1:])
+    assert same
+    if what == "k -inf":
+        k[0, at, 0], q64 = 0.0, q.astype(np.float64)
+        s = np.where(np.arange(n) == at, -np.inf, q64[:, 0] @ k[0].T.astype(np.float64) * 0.125)
+        s[np.arange(n)[None] > np.arange(n - m, n)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        err = rel(got[:, 0], p / p.sum(1, keepdims=True) @ v[0].astype(np.float64))
+        assert err < 2e-6
+    elif what[0] == "k":
+        none = (got[:, 0] == 0).all()
+        assert none
+    else:
+        bad = np.isnan(got[:, 0, 3]) if what == "v nan" else got[:, 0, 3] == np.inf
+        rest = [d for d in range(dh) if d != 3]
+        same = np.array_equal(got[:, 0, rest], plain[:, 0, rest])
+        assert bad.all() and same
+
+
 # one token, a query tile's segments on waves of their own, query tiles sharing key tiles, the general kernel
 @pytest.mark.parametrize("m,heads,dh", [(1, 2, 64), (3, 2, 64), (256, 12, 64), (40, 1, 32), (5, 1, 128), (1, 1, 128)])
 def test_attend_weights_of_large_scores(hip, m, heads, dh):
@@ -150,6 +188,45 @@ def test_attend_weights_of_large_scores(hip, m, heads, dh):
     hip.attend(dy.ptr, dq.ptr, dk.ptr, dv.ptr, **a)
     err = rel(dy.read(), attend64(q, k, v, **a))
     assert err < 5e-7
+
+
+@pytest.mark.parametrize("m,dh", [(1, 64), (40, 64), (40, 60), (5, 33), (3, 129)])
+@pytest.mark.parametrize("what", ["q", "k", "v", "s"])
+def test_gla_infinities(hip, m, dh, what):
+    """NaN and infinities come out where the oracle has them, the other elements within 2e-6."""
+    rng, heads = np.random.default_rng(m + dh), 2
+    q, k, v = (rng.standard_normal((m, heads, dh)).astype(np.float32) for _ in range(3))
+    s, dec, bias = (rng.standard_normal(n).astype(np.float32) for n in ((heads, dh, dh), (m, heads), heads))
+    if what == "s":
+        s[0, 3, 5] = np.inf
+    else:
+        dict(q=q, k=k, v=v)[what][m // 2, 0, 5] = np.nan
+    b = [hip.upload(t) for t in (s, q, k, v, dec, bias)]
+    dy = hip.alloc(q.size)
+    hip.gla(dy.ptr, *(t.ptr for t in b), m, heads, dh)
+    for got, want in zip((dy.read(), b[0].read()), O.gla(s, q, k, v, dec, bias, m, heads, dh)):
+        want = want.ravel()
+        fin = np.isfinite(want)
+        same = np.array_equal(got[~fin], want[~fin], equal_nan=True)
+        err = rel(got[fin], want[fin])
+        assert same and err < 2e-6
+
+
+@pytest.mark.parametrize("rows,cols,m", [(100, 768, 5), (100, 768, 20), (100, 768, 40), (100, 770, 5), (100, 770, 20),
+                                         (100, 770, 40), (100, 3072, 5), (9, 100, 33)])
+def test_linear_infinities(hip, rows, cols, m):
+    """An infinite weight reaches its row, an infinite input its token, NaN where both meet."""
+    rng = np.random.default_rng(rows + m)
+    w, x = (rng.standard_normal(s).astype(np.float32) for s in ((rows, cols), (m, cols)))
+    w[2, 37], w[4, 1], x[3, cols - 1] = np.inf, np.nan, -np.inf
+    dw, dx, dy = hip.upload(w), hip.upload(x), hip.alloc(rows * m)
+    hip.linear(dy.ptr, dw.ptr, rows, cols, dx.ptr, m)
+    with np.errstate(invalid="ignore"):
+        want = (x.astype(np.float64) @ w.T.astype(np.float64)).ravel()
+    got, fin = dy.read(), np.isfinite(want)
+    same = np.array_equal(got[~fin], want[~fin], equal_nan=True)
+    err = rel(got[fin], want[fin])
+    assert same and err < 2e-6
 
 
 @pytest.mark.parametrize("fp16", [False, True])

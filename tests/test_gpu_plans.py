@@ -215,3 +215,28 @@ def test_step_whose_capture_fails(hip):
     for n in want:
         assert np.array_equal(want[n], got[n]), n
     assert hip.graph_stats()["captured"] == after["captured"] + 1
+
+
+def test_more_lists_than_are_kept(hip):
+    """Forty lists in turn, four times over (32 are kept): each run's bits are its first run's."""
+    s = Lists(hip)
+    n = 40
+    s.buf("x", D), s.buf("w", D * D)
+    for i in range(n):
+        s.buf(f"y{i}", D)
+
+    def step(i):
+        hip.rope_table(s.cs.ptr, s.sn.ptr, s.inv.ptr, 3, 1, D // 2)
+        hip.linear(s[f"y{i}"], s["w"], D, D, s["x"], 1)
+        hip.add(s[f"y{i}"], s[f"y{i}"], s["x"], D - 4 * (i % 8))
+        hip.flush([b.ptr for b in s.bufs.values()])
+
+    want = {}
+    for b, v in s.first.items():
+        hip.upload_into(s.bufs[b], v)
+    for turn in range(4):
+        for i in range(n):
+            hip.upload_into(s.bufs[f"y{i}"], s.first[f"y{i}"])
+            step(i)
+            got = s.bufs[f"y{i}"].read()
+            assert np.array_equal(got, want.setdefault(i, got)), (turn, i)
