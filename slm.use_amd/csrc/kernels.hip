@@ -1437,11 +1437,12 @@ __device__ void gemm2_body(float* __restrict__ y, float* __restrict__ part,
 // slice of its columns at once, a slice a wave at a time: the wave's weights and tokens come
 // straight into registers (nothing is staged, no barrier until the slices are done), the slice
 // partials meet in LDS and one pass adds them in order. What bounds these shapes is latency, not
-// rate: the prompt GEMMs below walk a split's twelve slices one after another through LDS, a
+// rate: the prompt GEMMs above walk a split's twelve slices one after another through LDS, a
 // memory round trip each (a 21-token 2304 x 768 projection 20 us); here all twelve are in
 // flight together. Each workgroup reads all its tokens, so the GEMMs, whose tiles share
-// them, are the faster past 32 tokens and, for many rows, past 16 (few_tokens in runtime.cpp). 768 x 3072 at 5 tokens 13.8 -> 7.4 us (with the launch that adds its
-// four splits), 2304 x 768 5.3 -> 4.3; 2304 x 768 with the attention epilogue at 21 tokens 20 -> 7.
+// them, are the faster past 32 tokens and, for many rows, past 16 (few_tokens in runtime.cpp). 768 x
+// 3072 at 5 tokens 13.3 -> 6.8 us in a run of calls, 13.8 -> 8.3 among others (with the launch that adds
+// its four splits), 2304 x 768 5.3 -> 4.3; 2304 x 768 with the attention epilogue at 21 tokens 20 -> 7.
 // EPI 0: y [m][rows] (or, with several splits in blockIdx.z, part[split][m][rows]); rt rows a
 // tile (16, 8 or 4: a short matrix spreads over more CUs; the other MFMA rows are zeros).
 // EPI 1: the SiLU pair (tile rows i and i + 8 are gate and amp), as gemm2's SILU. EPI 2: the
@@ -1455,7 +1456,8 @@ __device__ __forceinline__ void linear_small_body(float* __restrict__ y, float* 
                              int cols, int m, int rt, GemmEpi ep = GemmEpi{}) {
     static_assert(!W16 || H, "fp16 weights run the fp16 chain");
     constexpr int RW = EPI == 3 ? 4 : 1, TR = 16 * RW, NTOK = 16 * NV;
-    constexpr int J = NV == 1 ? 3 : NV == 2 ? 2 : 1;  // slices in flight a wave (128 registers)
+    static_assert(NV == 1 || NV == 2, "up to 32 tokens");
+    constexpr int J = NV == 1 ? 3 : 2;  // slices in flight a wave (128 registers)
     extern __shared__ __attribute__((aligned(16))) float lds[];  // [slices][NTOK][TR], then [NTOK][TR + 1]
     int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int waves = blockDim.x >> 6, i = lane & 15, g = lane >> 4;
@@ -2097,7 +2099,9 @@ ATTN_PART(16)
 // workgroups of four waves share a CU, so one's copies and waits pass behind the others' tiles;
 // with all of a superblock staged at once (128 KB, one workgroup of 16 waves a CU) nothing
 // covered its copies and its fold. 256 queries, 12 heads of 64, a 4096-key window: 79.3 ->
-// 55.7 us a call with the combine, then 50.3 with exp2a (2 waves and 2 buffers 73.9, 4 and 3 56.4, 4 and 4 62.8).
+// 55.7 us a call with the combine (2 waves and 2 buffers 73.9, 4 and 3 56.4, 4 and 4 62.8), then 50.6 with
+// weights by exp2a.
+
 // Output dim of o[dt][r] in lane (i, g) of a prompt-attention wave. With DT = 4 the P·V MFMA
 // of block dt takes dims 4i + dt (A row i), so that the four values a lane needs of one key
 // are one 16-byte chunk (one LDS read per key instead of four); the accumulator then holds

@@ -72,8 +72,8 @@ def test_linear(hip, rows, cols, m):
 @pytest.mark.parametrize("rows,cols", [(768, 768), (6144, 768), (768, 3072), (97, 32), (40, 52),
                                        (64, 1600), (8192, 768), (2300, 768), (6150, 768)])
 def test_linear_same_bits_for_any_m(hip, rows, cols):
-    """The decode kernel (m <= 16) and the prompt kernels (m > 16, every row tile: 32, 64,
-    96 and 128 rows, ragged last tiles) run one MFMA chain."""
+    """The few-token kernels (to 16 tokens here) and the prompt GEMMs (256 tokens, every row tile: 32,
+    64, 96 and 128 rows, ragged last tiles) run one MFMA chain."""
     m = 256
     w = rnd(rows, cols, scale=0.02)
     x = rnd(m, cols)
