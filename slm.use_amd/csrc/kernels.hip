@@ -2748,7 +2748,7 @@ __device__ __forceinline__ bool attn_dec_body(float* __restrict__ part, const fl
             float muse = mnew == NEG_INF ? 0.0f : mnew;
             float alpha = exp2a(mo - muse);
             if (!any) continue;
-            if ((j >> 4) == st) pt[j & 15] = sv == NEG_INF ? 0.0f : weight(s, scale, muse);
+            if ((j >> 4) == st) pt[j & 15] = exp2a(ok ? fmaf(s, scale, -muse) : NEG_INF);  // weight(), 0 unseen
             float p[16];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
