@@ -2540,6 +2540,11 @@ struct Planner {
                     i += used;
                     continue;
                 }
+                if (!pend.empty()) {  // what was pending stands in its way: run that, then try again
+                    TRY(row_flush());
+                    TRY(flush_pending());
+                    continue;
+                }
             }
             // prompt rows: element-wise ops join a row chain; a split GEMM's fold starts one
             if (fuse && pend.empty() && !l2q && o.kind != OP_LINEAR && row_try(o)) {

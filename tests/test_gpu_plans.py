@@ -187,6 +187,25 @@ def test_second_matrix_with_an_epilogue_of_its_own(hip, kind, most):
     s.same(ops, most)
 
 
+def test_pending_op_in_a_matrix_launchs_way(hip):
+    """A pending op that reads what a matrix's epilogue writes runs first; the matrix keeps its
+    fusion (here a QKV input whose rotated q replaces the row a shift read)."""
+    s = Lists(hip)
+    s.buf("x", D), s.buf("prev", D), s.buf("sh", D), s.buf("w", 3 * D * D), s.buf("y", 3 * D), s.buf("kr", D)
+    s.buf("k", 8 * D, (1, 8, D)), s.buf("v", 8 * D, (1, 8, D))
+
+    def ops():
+        h = hip
+        h.shift(s["sh"], s["prev"], s["x"], 1, D)
+        h.linear(s["y"], s["w"], 3 * D, D, s["x"], 1)
+        h.rope(s["prev"], s["y"], s.cs.ptr, s.sn.ptr, 1, 1, D)
+        h.rope(s["kr"], s.at("y", D), s.cs.ptr, s.sn.ptr, 1, 1, D)
+        h.store(s["k"], s["kr"], 6, 1, 8, 1, D)
+        h.store(s["v"], s.at("y", 2 * D), 6, 1, 8, 1, D)
+
+    s.same(ops, 3)
+
+
 def test_step_whose_capture_fails(hip):
     """A list whose graph cannot be made has run all the same: no error, its state advanced once a
     run (a running sum, a ring), over replays of another list and after captures work again."""
