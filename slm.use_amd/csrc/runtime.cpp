@@ -1899,9 +1899,9 @@ struct Planner {
         // a second matrix on the same input (a global layer's q and kv, model.rs:493-494), unless
         // the ops after it are the epilogue of a launch of its own, which a pair has no place for
         bool pair = false;
-        bool own = (is(i + 2, OP_ROPE) && is(i + 3, OP_ROPE) && is(i + 4, OP_STORE) && is(i + 5, OP_STORE)) ||
-                   (is(i + 2, OP_L2NORM) && is(i + 3, OP_L2NORM) && is(i + 4, OP_LINEAR)) ||
-                   (is(i + 2, OP_ARGMAX) && ops[i + 2].p[1] == ops[i + 1].p[0]);
+        bool own = is(i + 1, OP_LINEAR) && i + 2 < ops.size() && ops[i + 2].p[1] == ops[i + 1].p[0] &&
+                   ((is(i + 2, OP_ROPE) && is(i + 3, OP_ROPE) && is(i + 4, OP_STORE) && is(i + 5, OP_STORE)) ||
+                    (is(i + 2, OP_L2NORM) && is(i + 3, OP_L2NORM) && is(i + 4, OP_LINEAR)) || is(i + 2, OP_ARGMAX));
         if (s0.epi == EPI_PLAIN && nseg == 1 && nsplit == 1 && is(i + 1, OP_LINEAR) && !own && *extras < most) {
             const Op& D = ops[i + 1];
             if (D.n[2] == 1 && D.p[2] == x && D.n[1] == cols && D.n[0] >= 1 && D.n[0] <= (int64_t)1 << 26 &&

@@ -154,7 +154,7 @@ def test_lists_with_an_extra_that_cannot_join(hip, kind, most):
     s.same(ops, most)
 
 
-@pytest.mark.parametrize("kind,most", [("rope", 2), ("l2norm", 3), ("pick", 2)])
+@pytest.mark.parametrize("kind,most", [("rope", 2), ("l2norm", 3), ("pick", 2), ("rope of another", 5)])
 def test_second_matrix_with_an_epilogue_of_its_own(hip, kind, most):
     """A matrix whose own launch takes the ops after it (rope and ring stores, the l2norms of a
     linear-attention input, a pick) is not paired with the matrix before it."""
@@ -174,6 +174,12 @@ def test_second_matrix_with_an_epilogue_of_its_own(hip, kind, most):
             h.rope(s["kr"], s.at("y", D), s.cs.ptr, s.sn.ptr, 1, 1, D)
             h.store(s["k"], s["kr"], 6, 1, 8, 1, D)
             h.store(s["v"], s.at("y", 2 * D), 6, 1, 8, 1, D)
+        elif kind == "rope of another":  # (these two are a pair)
+            h.linear(s["y"], s["w"], 3 * D, D, s["n"], 1)
+            h.rope(s["q"], s["s"], s.cs.ptr, s.sn.ptr, 1, 1, D)
+            h.rope(s["kr"], s.at("s", D), s.cs.ptr, s.sn.ptr, 1, 1, D)
+            h.store(s["k"], s["kr"], 6, 1, 8, 1, D)
+            h.store(s["v"], s.at("s", 2 * D), 6, 1, 8, 1, D)
         elif kind == "l2norm":
             h.linear(s["y"], s["w"], 4 * D, D, s["n"], 1)
             h.l2norm(s["q"], s["y"], 1, D)
