@@ -606,9 +606,8 @@ void drop_graphs(slm_hip* c) {
 // per-op lowering (the unfused kernels)
 // ---------------------------------------------------------------------------------------
 
-// The pipelined prompt GEMM's row tile: the one that leaves the busiest CU the least work —
-// rows per tile times the workgroups a CU runs (32-row tiles of four waves go two to a CU,
-// the others one) — the larger tile on a tie.
+// The tile rows the busiest CU runs of a pipelined prompt GEMM with t rows a tile: rows per tile
+// times the workgroups a CU runs (32-row tiles of four waves go two to a CU, the others one).
 int64_t gemm2_work(int64_t t, int64_t rows, int64_t m, int64_t ns) {
     int64_t wgs = ((rows + t - 1) / t) * ((m + 63) / 64) * ns;
     int64_t per_cu = t == 32 ? 2 : 1;
@@ -616,6 +615,7 @@ int64_t gemm2_work(int64_t t, int64_t rows, int64_t m, int64_t ns) {
     int64_t sharing = std::min<int64_t>(per_cu, (wgs + CU_COUNT - 1) / CU_COUNT);
     return rounds * t * sharing;
 }
+// Its row tile: the one that leaves the busiest CU the least work, the larger tile on a tie.
 int gemm2_bm(int64_t rows, int64_t m, int64_t ns) {
     int bm = 32;
     int64_t best = -1;
